@@ -9,339 +9,363 @@
 // Weights: row n, weight k is bit k % 32 of sign word [n][k / 32] (set = +1, clear = -1) times the
 // f32 scale [n][k / 128] (shaders/matmul_split_sg.wgsl:24-35).
 //
-//   rows    a wave computes kGemvRW output rows; a lane owns one 32-weight word of each row per
-//           2048-weight tile of K. Rows up to kLutMaxK long (the Qwen3-8B qkv and o_proj): the
-//           workgroup first tabulates, for every word of x and each of its 8 nibbles, the 16
-//           signed sums of the nibble's 4 x values (64 KB of LDS at K = 4096); a word's signed sum
-//           is then 8 table reads (indexed by the word's nibbles) and 7 adds instead of 32
-//           sign flips and adds. Longer rows: the lane holds the 32 x values under its word
-//           (eight 16-byte loads from LDS or memory, reused by the wave's rows) and the word's
-//           signs flip their sign bits (one xor each), four partial sums per word. Either way
-//           times the word's block scale; a DPP / permlane wave sum finishes the row. With the
-//           table (at most two tiles) x is loaded first and both tiles' weights are issued
-//           before the table is built, so it is built under their latency; longer
-//           rows keep two tiles' loads (the rows' words and scales, x) in flight, the next tile
-//           issued before the current one's arithmetic. The residual is loaded at the start.
+//   contraction  the signed sums of a row's 128-weight blocks run on the int8 matrix cores
+//           (v_mfma_i32_16x16x64_i8), exactly: x becomes a 28-bit fixed-point number over its
+//           block's largest power of two, in four signed int8 digits, and the integer sums are
+//           scaled back per block. One sign word is the weight operand of two MFMAs after one
+//           AND a dword: a byte masked to bit j is 0 or 2^j (-128 for j = 7), and x is prepared
+//           with the factor 2^(7-j) for those weights, so no bit is shifted to its place (bits
+//           0-3 after one shift by 4). sum (2b - 1) x = sum 2b x - sum x: the second sum is the
+//           integers' start, got from the same MFMAs over all-ones weights.
+//           Against the table of signed 4-term sums it replaces (8 LDS reads and 24 VALU a word,
+//           16 K bytes of table built by every workgroup; rows past 4096 weights 32 sign flips and
+//           adds) a word costs 9 ANDs and shifts and a quarter of two MFMAs. us a launch, graph
+//           replays over 36 weights (read floor of the same bytes): gate | up 24576 x 4096 10.5 ->
+//           6.8 (4.7), down 4096 x 12288 10.3 -> 5.45 (3.6), o_proj 4096 x 4096 3.48 -> 3.3 (2.9),
+//           qkv + prologue 4.8 as before (3.05; K = 2560: 4.72 -> 4.46). Bound by the latency of
+//           x, its conversion (about 100 VALU a wave), then the weights' arrival.
+//   precision  x is rounded to 2^-28 of its block's largest magnitude's power of two, the block
+//           sums are exact, f32 from there on: error against 64 bits 7e-8 relative, 9e-8 for the
+//           f32 sums it replaces. A block with an infinity or a NaN is summed directly in f32.
+//   lanes   a 16-row tile x 4 blocks (512 weights) a step: lane 16 g + n holds the four words of
+//           row n, block g (one 16-byte load), so the MFMA's four k groups are the four blocks.
+//           The x operand is block diagonal: its row 4 g + p holds digit p of block g in k group
+//           g and zeros elsewhere, so lane 16 g + n gets back row n's sum over block g (a digit a
+//           register), which its own scale multiplies: 7 VALU for 64 block sums.
+//   split   the waves of a workgroup split K (steps of 512; each prepares only its own x, in
+//           registers), every wave runs the workgroup's T tiles over its part; the parts meet in
+//           LDS. All loads of a wave's step are in flight before x is converted. How K is split
+//           depends on K alone, so a row's sum has the same bits in every kernel and grid.
 //   fused   the qkv kernel's workgroups own 32 rows of one head; all but the head's last one
 //           store their raw rows into the cache's gather buffer (the XCD's L2 when the head's
 //           workgroups share an XCD) and are done; the last one polls them in (no arrival
-//           ticket, no store acknowledgement: 6.66 -> 5.9 us at the 8B shape), writes the
-//           empty markers back at once, normalizes and ropes the head (Q -> q_out; K -> the
-//           cache row, unroped in sink mode) or stores it (V), with the fused prologue's row
-//           arithmetic (bg_qkrow.h; the rope partner by a lane exchange). Markers first, the
-//           lane exchange and x before the weights: 5.65 -> 5.30 us; 24-row workgroups over
-//           every CU (a workgroup may hold the end of one head and the start of the next): 5.19;
-//           the poll before the finisher's barrier: 4.85.
-#include <map>
-#include <mutex>
-
+//           ticket, no store acknowledgement), writes the empty markers back at once, normalizes
+//           and ropes the head (Q -> q_out; K -> the cache row, unroped in sink mode) or stores it
+//           (V), with the fused prologue's row arithmetic (bg_qkrow.h; the rope partner by a lane
+//           exchange).
 #include "bg_kernels.h"
 #include "bg_qkrow.h"
 
 namespace bg {
 
-// 2 rows a wave, 8 waves a workgroup (16 rows): o_proj at the 8B shape 3.8 us against 4.4 with 4
-// rows on 4 waves (the same rows a workgroup, twice the waves to cover the loads' latency), 4.3
-// with 4 rows on 8 waves
-constexpr int kGemvRW = 2;
-constexpr int kGemvWaves = 8;
-constexpr int kGemvThreads = 64 * kGemvWaves;
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
-// One 2048-weight tile of a wave's rows: the lane's sign word (word 64t + l) and block scale of
-// each row and the 32 x values under the word.
-template <int RW>
-struct GemvTile {
-  uint32_t word[RW];
-  float sc[RW];
-  float xv[32];
+constexpr int kTileRows = 16;    // rows of an MFMA tile
+constexpr int kStepK = 512;      // weights a tile and step: 4 blocks of 128
+constexpr int kGemvMaxWaves = 16;
+
+// How K is split over a workgroup's waves: wave w takes steps [w per, (w + 1) per). One step a wave
+// up to 16 waves; longer rows 2 and more (12288 weights on 12 waves of 2 steps 5.4 us, on 8 waves
+// of 3 5.8 us, 4096 rows).
+struct GemvSplit {
+  int steps, per, waves;
+};
+__host__ __device__ inline GemvSplit gemv_split(int K) {
+  GemvSplit s;
+  s.steps = (K + kStepK - 1) / kStepK;
+  s.per = (s.steps + kGemvMaxWaves - 1) / kGemvMaxWaves;
+  s.waves = (s.steps + s.per - 1) / s.per;
+  return s;
+}
+
+// A wave's x digits in LDS: 16 rows (block g, digit p) of 128 bytes (digit byte i of weight order
+// below), 16 bytes of pad a row so that the 16 lanes reading one column of them fall on distinct
+// banks, then 128 bytes of zeros for the lanes off the operand's block diagonal.
+constexpr int kDigitRow = 144;
+constexpr int kDigitZero = 16 * kDigitRow;
+constexpr int kDigitBytes = kDigitZero + 128;
+
+// A step's weights of T tiles and its x values, as loaded
+template <int T>
+struct GemvStep {
+  u32x4_t word[T];
+  float sc[T];
+  float2 x[4];
 };
 
-// x staged in LDS by the workgroup: word w's 32 values at float offset 36 w (4 floats of pad
-// per word keep the lanes' 16-byte reads of consecutive words on different banks)
-constexpr int kXPad = 36;
-constexpr int kGemvLdsMaxK = 12288;  // 54 KB of LDS; longer rows read x from global memory
-
-// Where a lane finds the x values under its words: kXGlobal (memory), kXLds (x staged in LDS),
-// kXLut (the nibble table below; K <= kLutMaxK)
-constexpr int kXGlobal = 0, kXLds = 1, kXLut = 2;
-constexpr int kLutMaxK = 4096;  // 16 K bytes of LDS: 64 KB at the limit
-
-__host__ __device__ constexpr size_t gemv_lut_bytes(int K) { return (size_t)K * 16; }
-
-// The nibble table: lut[(16 g + e) W + w] = sum over k < 4 of (bit k of e set ? +x : -x) of
-// x[32 w + 4 g + k], summed as (k0, k1) + (k2, k3): every signed combination of a nibble's four
-// x values (bit set = weight +1, as in the word loop). W-fastest, so the lanes' reads (one word
-// each) fall on distinct banks. The NT threads of the workgroup build it (ceil(8 K / 32 / NT)
-// (word, nibble) pairs each at most) in two parts: the x loads are issued before the weight loads
-// (vector-memory waits retire in issue order, so the build then waits for x alone and runs under
-// the weights' latency), the table is written after them, then a barrier.
-template <int NT>
-struct LutX {
-  static constexpr int kPairs = (8 * (kLutMaxK / 32) + NT - 1) / NT;
-  float4 v[kPairs];
-};
-// pair i = g W + w (i < 8 W <= 1024): g = floor(i * ceil(2^20 / W) / 2^20), exact for W < 1000
-__device__ __forceinline__ int lut_pair_g(int i, unsigned inv_w) { return (int)(__umul24((unsigned)i, inv_w) >> 20); }
-template <int NT>
-__device__ __forceinline__ void gemv_lut_load(const float* __restrict__ x, int K, LutX<NT>& X) {
-  const int W = K >> 5;
-  const unsigned inv_w = ((1u << 20) + W - 1) / W;
-#pragma unroll
-  for (int j = 0; j < LutX<NT>::kPairs; j++) {
-    const int i = threadIdx.x + NT * j;
-    const int ic = i < 8 * W ? i : 8 * W - 1;  // unconditional load, as for the weights
-    const int g = lut_pair_g(ic, inv_w), w = ic - g * W;
-    X.v[j] = *(const float4*)(x + 32 * w + 4 * g);
-  }
-}
-template <int NT>
-__device__ __forceinline__ void gemv_lut_write(const LutX<NT>& X, float* lut, int K) {
-  const int W = K >> 5;
-  const unsigned inv_w = ((1u << 20) + W - 1) / W;
-#pragma unroll
-  for (int j = 0; j < LutX<NT>::kPairs; j++) {
-    const int i = threadIdx.x + NT * j;
-    if (i < 8 * W) {
-      const int g = lut_pair_g(i, inv_w), w = i - g * W;
-      const float4 v = X.v[j];
-      const float a[4] = {-v.x - v.y, v.x - v.y, v.y - v.x, v.x + v.y};
-      const float b[4] = {-v.z - v.w, v.z - v.w, v.w - v.z, v.z + v.w};
-      float* d = lut + (size_t)(16 * g) * W + w;
-#pragma unroll
-      for (int e = 0; e < 16; e++) d[(size_t)e * W] = a[e & 3] + b[e >> 2];
-    }
-  }
-  __syncthreads();
-}
-// BF: every load unconditional (clamped address, the value zeroed after), so no branch: the wait
-// counts stay exact and a later wait for loads issued before these does not drain them (the
-// table build then waits for its x loads alone); otherwise rows past the end are not loaded
-template <int RW, bool BF = false>
-__device__ __forceinline__ void gemv_load_w(GemvTile<RW>& T, int W, int NB, const uint32_t* __restrict__ sign,
-                                            const float* __restrict__ scales, int n0, int n_rows, int t, int lane) {
-  const int w = 64 * t + lane;
-  const bool ok = w < W;
-  const int wc = ok ? w : W - 1;
-#pragma unroll
-  for (int r = 0; r < RW; r++) {
-    const int n = n0 + r;
-    const bool v = ok && n < n_rows;
-    if constexpr (BF) {
-      const int nc = n < n_rows ? n : n_rows - 1;
-      const uint32_t wd = sign[(size_t)nc * W + wc];
-      const float sc = scales[(size_t)nc * NB + (wc >> 2)];
-      T.word[r] = v ? wd : 0u;
-      T.sc[r] = v ? sc : 0.0f;
-    } else {
-      T.word[r] = v ? sign[(size_t)n * W + w] : 0u;
-      T.sc[r] = v ? scales[(size_t)n * NB + (w >> 2)] : 0.0f;
-    }
-  }
-}
-
-template <int RW, int XM>
-__device__ __forceinline__ void gemv_load_x(GemvTile<RW>& T, const float* __restrict__ x, const float* xs, int W, int t,
-                                            int lane) {
-  if constexpr (XM == kXLut) return;  // the table holds x
-  const int w = 64 * t + lane;
-  const bool ok = w < W;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    float4 f;
-    if constexpr (XM == kXLds) f = ok ? *(const float4*)(xs + kXPad * w + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
-    else f = ok ? *(const float4*)(x + 32 * w + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
-    T.xv[4 * j] = f.x;
-    T.xv[4 * j + 1] = f.y;
-    T.xv[4 * j + 2] = f.z;
-    T.xv[4 * j + 3] = f.w;
-  }
-}
-
-template <int RW, int XM, bool BF>
-__device__ __forceinline__ void gemv_load(GemvTile<RW>& T, const float* __restrict__ x, const float* xs, int W, int NB,
-                                          const uint32_t* __restrict__ sign, const float* __restrict__ scales,
-                                          int n0, int n_rows, int t, int lane) {
-  gemv_load_w<RW, BF>(T, W, NB, sign, scales, n0, n_rows, t, lane);
-  gemv_load_x<RW, XM>(T, x, xs, W, t, lane);
-}
-
-// stage x[K] into xs (the whole workgroup, coalesced 16-byte loads), then a barrier
-__device__ __forceinline__ void gemv_stage_x(const float* __restrict__ x, float* xs, int K) {
-  for (int i = threadIdx.x; i < K / 4; i += blockDim.x) {
-    const float4 f = *(const float4*)(x + 4 * i);
-    *(float4*)(xs + kXPad * (i >> 3) + 4 * (i & 7)) = f;
-  }
-  __syncthreads();
-}
-
-template <int RW, int XM>
-__device__ __forceinline__ void gemv_accumulate(const GemvTile<RW>& T, float (&acc)[RW], const float* lut, int W, int t,
-                                                int lane) {
-  if constexpr (XM == kXLut) {
-    // a lane past the last word reads word W-1's entries, weighted by its zero scale; entry
-    // (g, e) of the lane's word at byte (16 g + e) 4W + 4w (24-bit products: the table is 64 KB)
-    const int w = min(64 * t + lane, W - 1);
-    const unsigned W4 = 4u * (unsigned)W;
-    const char* rowg[8];
-#pragma unroll
-    for (int g = 0; g < 8; g++) rowg[g] = (const char*)lut + 4 * w + __umul24(16u * g, W4);
-#pragma unroll
-    for (int r = 0; r < RW; r++) {
-      const uint32_t wd = T.word[r];
-      float l[8];
-#pragma unroll
-      for (int g = 0; g < 8; g++) l[g] = *(const float*)(rowg[g] + __umul24(__builtin_amdgcn_ubfe(wd, 4 * g, 4), W4));
-      acc[r] = fmaf(((l[0] + l[1]) + (l[2] + l[3])) + ((l[4] + l[5]) + (l[6] + l[7])), T.sc[r], acc[r]);
-    }
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < RW; r++) {
-    // clear bit i -> weight -1: flip the sign bit of x_i
-    const uint32_t nw = ~T.word[r];
-    float p[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int i = 0; i < 32; i++) p[i & 3] += __uint_as_float(__float_as_uint(T.xv[i]) ^ ((nw << (31 - i)) & 0x80000000u));
-    acc[r] = fmaf((p[0] + p[1]) + (p[2] + p[3]), T.sc[r], acc[r]);
-  }
-}
-
-// totals of rows n0 .. n0 + RW - 1 (rows >= n_rows give 0); every lane holds every total. Two
-// tiles are in flight: the next tile's loads are issued before the current tile's arithmetic
-// (a uniform trip count, so the compiler keeps them outstanding across the loop head).
-// (the caller issues tile 0's weight loads into A, then stages x or builds the table, then calls
-// this; xs is the staged x or the table)
-template <int RW, int XM, bool BF>
-__device__ inline void gemv_rows(GemvTile<RW>& A, const float* __restrict__ x, const float* xs, int K,
-                                 const uint32_t* __restrict__ sign, const float* __restrict__ scales, int n0, int n_rows,
-                                 int lane, float (&tot)[RW]) {
+// x first: it is needed first, and vector-memory waits retire in issue order. Every load is
+// unconditional (clamped to the last block; past the end x and the scales are zeroed at their use,
+// since a change here would wait for the loads).
+template <int T>
+__device__ __forceinline__ void gemv_load(GemvStep<T>& S, const float* __restrict__ x, int K,
+                                          const uint32_t* __restrict__ sign, const float* __restrict__ scales, int n0,
+                                          int n_rows, int step, int lane) {
   const int W = K >> 5, NB = K >> 7;
-  const int n_tiles = (W + 63) >> 6;
-  float acc[RW];
+  const int g = lane >> 4, l = lane & 15;
+  const int b = 4 * step + g, bc = b < NB ? b : NB - 1;
+  // lane l of group g prepares weights 32 (l >> 2) + 8 t + 4 ((l >> 1) & 1) + 2 (l & 1) + {0, 1}
+  // of block b, t = 0..3
+  const float* xb = x + 128 * bc + 32 * (l >> 2) + 2 * (l & 3);
 #pragma unroll
-  for (int r = 0; r < RW; r++) acc[r] = 0.0f;
-  GemvTile<RW> B;
-  gemv_load_x<RW, XM>(A, x, xs, W, 0, lane);
-  int t = 0;
-  for (; t + 2 <= n_tiles; t += 2) {
-    gemv_load<RW, XM, BF>(B, x, xs, W, NB, sign, scales, n0, n_rows, t + 1, lane);
-    gemv_accumulate<RW, XM>(A, acc, xs, W, t, lane);
-    if (t + 2 < n_tiles) gemv_load<RW, XM, BF>(A, x, xs, W, NB, sign, scales, n0, n_rows, t + 2, lane);
-    gemv_accumulate<RW, XM>(B, acc, xs, W, t + 1, lane);
+  for (int t = 0; t < 4; t++) S.x[t] = *(const float2*)(xb + 8 * t);
+  __builtin_amdgcn_sched_barrier(0);  // the loads keep this order (tile t's wait covers tiles 0..t)
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    const int n = n0 + kTileRows * t + l, nc = n < n_rows ? n : n_rows - 1;
+    S.word[t] = *(const u32x4_t*)(sign + (size_t)nc * W + 4 * bc);
+    S.sc[t] = scales[(size_t)nc * NB + bc];
+    __builtin_amdgcn_sched_barrier(0);
   }
-  if (t < n_tiles) gemv_accumulate<RW, XM>(A, acc, xs, W, t, lane);
-#pragma unroll
-  for (int r = 0; r < RW; r++) tot[r] = wave_sum(acc[r]);
 }
 
-// rows at most kLutMaxK long: the totals of the (at most) two tiles A (tile 0) and B (tile 1),
-// both loaded before the table was written
-template <int RW>
-__device__ __forceinline__ void gemv_lut_rows(const GemvTile<RW>& A, const GemvTile<RW>& B, const float* lut, int W,
-                                              int lane, float (&tot)[RW]) {
-  float acc[RW];
-#pragma unroll
-  for (int r = 0; r < RW; r++) acc[r] = 0.0f;
-  gemv_accumulate<RW, kXLut>(A, acc, lut, W, 0, lane);
-  if (W > 64) gemv_accumulate<RW, kXLut>(B, acc, lut, W, 1, lane);
-#pragma unroll
-  for (int r = 0; r < RW; r++) tot[r] = wave_sum(acc[r]);
+// dword j of the weight operand's half h: bit 4 + j of each byte of the word shifted by 4 h
+__device__ __forceinline__ i32x4_t weight_operand(uint32_t w) {
+  return i32x4_t{(int)(w & 0x10101010u), (int)(w & 0x20202020u), (int)(w & 0x40404040u), (int)(w & 0x80808080u)};
 }
 
-template <int XM>
-__global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvArgs a) {
-  extern __shared__ __align__(16) float xs[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int N = a.N0 + a.N1 + a.N2;
-  const int n0 = (blockIdx.x * kGemvWaves + wave) * kGemvRW;
-  // lane r < kGemvRW stores row n0 + r: its residual and the first tile's weights are loaded
-  // before x is staged
-  LutX<kGemvThreads> X;
-  if constexpr (XM == kXLut) gemv_lut_load<kGemvThreads>(a.x, a.K, X);
-  const float res = (a.resid && lane < kGemvRW && n0 + lane < N) ? a.resid[n0 + lane] : 0.0f;
-  GemvTile<kGemvRW> A;
-  gemv_load_w<kGemvRW, XM == kXLut>(A, a.K >> 5, a.K >> 7, a.sign, a.scales, n0, N, 0, lane);
-  float tot[kGemvRW];
-  if constexpr (XM == kXLut) {
-    // K <= kLutMaxK: at most two tiles, both issued before the table is written, so the second
-    // tile's latency runs under the build too (o_proj at the 8B shape: 3.77 -> 3.60 us)
-    const int W = a.K >> 5;
-    GemvTile<kGemvRW> B;
-    gemv_load_w<kGemvRW, true>(B, W, a.K >> 7, a.sign, a.scales, n0, N, 1, lane);
-    gemv_lut_write<kGemvThreads>(X, xs, a.K);
-    if (n0 >= N) return;  // wave-uniform
-    gemv_lut_rows<kGemvRW>(A, B, xs, W, lane, tot);
-  } else {
-    if constexpr (XM == kXLds) gemv_stage_x(a.x, xs, a.K);
-    if (n0 >= N) return;  // wave-uniform
-    gemv_rows<kGemvRW, XM, false>(A, a.x, xs, a.K, a.sign, a.scales, n0, N, lane, tot);
-  }
+// The x operand of a step: digits a[2 w + h] for sign word w and half h (weights 32 w + 8 t + 4 (1
+// - h) + j, byte t of dword j), what the sums start from, and each lane's block exponent.
+struct GemvX {
+  i32x4_t a[8];
+  i32x4_t c;  // minus the half sums over all-ones weights, what the sums start from
+  int exp;    // block sum = integer sum x 2^exp
+  bool in;    // the lane's block lies in the row
+  bool bad;   // the lane's block holds an infinity or a NaN
+};
+
+// floor(v + 0.5) in one instruction
+__device__ __forceinline__ int round_i32(float v) {
+  int r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
+template <int T>
+__device__ __forceinline__ void gemv_prepare(GemvX& X, const GemvStep<T>& S, int K, int step, char* dig, int lane) {
+  const int g = lane >> 4, l = lane & 15;
+  X.in = 4 * step + g < (K >> 7);
+  // largest magnitude of the lane's block (over its 16 lanes), as bits: infinities and NaN largest
+  uint32_t mb = 0;
 #pragma unroll
-  for (int r = 0; r < kGemvRW; r++) {
-    const int n = n0 + r;
-    if (lane == r && n < N) {
-      const float y = a.resid ? tot[r] + res : tot[r];
-      if (n < a.N0) a.out0[n] = y;
-      else if (n < a.N0 + a.N1) a.out1[n - a.N0] = y;
-      else a.out2[n - a.N0 - a.N1] = y;
+  for (int t = 0; t < 4; t++)
+    mb = max(max(mb, __float_as_uint(S.x[t].x) & 0x7fffffffu), __float_as_uint(S.x[t].y) & 0x7fffffffu);
+  auto dppmax = [&](auto ctrl) {
+    mb = max(mb, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mb, decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  dppmax(std::integral_constant<int, kDppXor1>{});
+  dppmax(std::integral_constant<int, kDppXor2>{});
+  dppmax(std::integral_constant<int, kDppHalfMirror>{});
+  dppmax(std::integral_constant<int, kDppMirror>{});
+  X.bad = X.in && mb >= 0x7f800000u;
+  const int e = (int)(mb >> 23) - 126;  // |x| < 2^e
+  X.exp = e - 33;
+  // weights whose sign bit is masked at bit 4 + j carry 2^(4 + j): x x 2^(27 - e) x 2^(3 - j),
+  // at most 2^30; bit 7 reads as -128. Past the row's end everything becomes 0. (An infinity or
+  // NaN leaves some integer: only its own block sees it, and that one is summed again in f32.)
+  const int jp = 2 * (l & 1);
+  const int h = 1 - ((l >> 1) & 1);
+  uint32_t y[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int sh = X.in ? 30 - e - (jp + u) : -1024;
+    const uint32_t flip = jp + u == 3 ? 0x80000000u : 0u;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const uint32_t v = __float_as_uint(u == 0 ? S.x[t].x : S.x[t].y);
+      const int q = round_i32(ldexpf(__uint_as_float(u == 0 ? v : v ^ flip), sh));
+      y[u][t] = ((uint32_t)q + 0x80808080u) ^ 0x80808080u;  // signed base-256 digits
     }
   }
+  // 4 x 4 byte transposes: dword of digit p = byte p of y[.][0..3]
+  char* row = dig + (4 * g) * kDigitRow + (2 * (l >> 2) + h) * 16 + 4 * jp;
+  uint32_t d[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const uint32_t p01 = __builtin_amdgcn_perm(y[u][1], y[u][0], 0x05010400u);  // y0.b0 y1.b0 y0.b1 y1.b1
+    const uint32_t p23 = __builtin_amdgcn_perm(y[u][3], y[u][2], 0x05010400u);
+    const uint32_t q01 = __builtin_amdgcn_perm(y[u][1], y[u][0], 0x07030602u);  // bytes 2, 3
+    const uint32_t q23 = __builtin_amdgcn_perm(y[u][3], y[u][2], 0x07030602u);
+    d[u][0] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+    d[u][1] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
+    d[u][2] = __builtin_amdgcn_perm(q23, q01, 0x05040100u);
+    d[u][3] = __builtin_amdgcn_perm(q23, q01, 0x07060302u);
+  }
+  // the reads of the step before are done (their MFMAs have used them); the wave's own LDS
+  // accesses complete in order
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int p = 0; p < 4; p++) *(uint2*)(row + p * kDigitRow) = make_uint2(d[0][p], d[1][p]);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // row m = l of the operand: digit l & 3 of block l >> 2, nonzero in that block's k group only
+  const char* src = dig + ((l >> 2) == g ? l * kDigitRow : kDigitZero);
+#pragma unroll
+  for (int i = 0; i < 8; i++) X.a[i] = *(const i32x4_t*)(src + 16 * i);
+  // minus half of the sums over all-ones weights (those are even: every weight byte is)
+  i32x4_t f[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+  for (int i = 0; i < 8; i++) f[i & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(X.a[i], weight_operand(~0u), f[i & 1], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; i++) X.c[i] = -((f[0][i] + f[1][i]) >> 1);
 }
 
-// the LDS a kernel may take beyond the default (at most 64 KB of table plus a few static arrays),
-// set once per kernel
-static hipError_t gemv_allow_lds(const void* fn, size_t bytes) {
-  static std::mutex mu;
-  static std::map<const void*, size_t> allowed;
-  std::lock_guard<std::mutex> lock(mu);
-  size_t& a = allowed[fn];
-  if (bytes <= a) return hipSuccess;
-  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e == hipSuccess) a = bytes;
-  return e;
+// the lane's block sum directly in f32, for a block that holds an infinity or a NaN
+__device__ __noinline__ float gemv_block_f32(const float* __restrict__ xb, u32x4_t word) {
+  float s = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    const uint32_t nw = ~word[w];
+#pragma unroll 1
+    for (int i = 0; i < 32; i++) s += __uint_as_float(__float_as_uint(xb[32 * w + i]) ^ ((nw << (31 - i)) & 0x80000000u));
+  }
+  return s;
+}
+
+template <int T>
+__device__ __forceinline__ void gemv_accumulate(float (&acc)[T], const GemvStep<T>& S, const GemvX& X,
+                                                const float* __restrict__ x, int K, int step, int lane) {
+  float s[T];
+  // two tiles at a time, or the two halves of one: independent MFMA chains (exact integer sums, so
+  // their order does not matter). A single tile does not wait for the start values either.
+#pragma unroll
+  for (int t0 = 0; t0 < T; t0 += 2) {
+    const bool pair = t0 + 1 < T;
+    const i32x4_t zero = {0, 0, 0, 0};
+    i32x4_t d[2] = {T == 1 ? zero : X.c, pair ? X.c : zero};
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int u = 0; u < (pair ? 2 : 1); u++) {
+        const uint32_t w = S.word[t0 + u][i >> 1];
+        i32x4_t& dd = d[pair ? u : i & 1];
+        dd = __builtin_amdgcn_mfma_i32_16x16x64_i8(X.a[i], weight_operand(i & 1 ? w << 4 : w), dd, 0, 0, 0);
+      }
+    if (!pair) d[0] += T == 1 ? d[1] + X.c : d[1];
+#pragma unroll
+    for (int u = 0; u < (pair ? 2 : 1); u++) {
+      // digits 0, 1 and 2, 3 join as integers (|d| <= 2^21, so below 2^30), then in f32
+      const float lo = (float)(d[u][0] + (d[u][1] << 8)), hi = (float)(d[u][2] + (d[u][3] << 8));
+      s[t0 + u] = ldexpf(fmaf(hi, 65536.0f, lo), X.exp);
+    }
+  }
+  if (__any(X.bad)) {
+    const int b = min(4 * step + (lane >> 4), (K >> 7) - 1);
+#pragma unroll
+    for (int t = 0; t < T; t++)
+      if (X.bad) s[t] = gemv_block_f32(x + 128 * b, S.word[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < T; t++) acc[t] = fmaf(s[t], X.in ? S.sc[t] : 0.0f, acc[t]);
+}
+
+// One wave's part of the workgroup's rows n0 .. n0 + 16 T - 1: the sums over its steps into
+// red[wave][row]. PER: the steps a wave takes when that is at most 2 (K <= 16384): all their
+// loads are issued before the first x is converted; 0: any number, the next step's loads issued
+// before this one's x is converted. dig: the wave's kDigitBytes of LDS.
+template <int T, int PER>
+__device__ __forceinline__ void gemv_part(const float* __restrict__ x, int K, const uint32_t* __restrict__ sign,
+                                          const float* __restrict__ scales, int n0, int n_rows, int wave, int lane,
+                                          char* dig, float* red) {
+  const GemvSplit sp = gemv_split(K);
+  const int s0 = wave * sp.per, s1 = min(s0 + sp.per, sp.steps);
+  constexpr int NB = PER ? PER : 2;
+  GemvStep<T> S[NB];
+#pragma unroll
+  for (int i = 0; i < (PER ? PER : 1); i++) gemv_load<T>(S[i], x, K, sign, scales, n0, n_rows, min(s0 + i, s1 - 1), lane);
+  if (lane < 8) *(uint4*)(dig + kDigitZero + 16 * lane) = make_uint4(0, 0, 0, 0);
+  float acc[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) acc[t] = 0.0f;
+  GemvX X;
+  auto step = [&](const GemvStep<T>& A, int s) {
+    gemv_prepare<T>(X, A, K, s, dig, lane);
+    gemv_accumulate<T>(acc, A, X, x, K, s, lane);
+  };
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (i == 0 || s0 + i < s1) step(S[i], s0 + i);
+  } else {
+    for (int s = s0; s < s1; s += 2) {
+      gemv_load<T>(S[1], x, K, sign, scales, n0, n_rows, min(s + 1, s1 - 1), lane);
+      step(S[0], s);
+      if (s + 1 >= s1) break;
+      gemv_load<T>(S[0], x, K, sign, scales, n0, n_rows, min(s + 2, s1 - 1), lane);
+      step(S[1], s + 1);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    float2 r = pair16(acc[t]);
+    r = pair32(r.x + r.y);
+    if (lane < kTileRows) red[wave * (kTileRows * T) + kTileRows * t + lane] = r.x + r.y;
+  }
+}
+
+// row r of the workgroup: its parts in wave order (after the barrier)
+template <int T, int NW>
+__device__ __forceinline__ float gemv_row(const float* red, int r, int waves) {
+  float p[NW];
+#pragma unroll
+  for (int w = 0; w < NW; w++) p[w] = red[min(w, waves - 1) * (kTileRows * T) + r];
+  float y = p[0];
+#pragma unroll
+  for (int w = 1; w < NW; w++) y += w < waves ? p[w] : 0.0f;
+  return y;
+}
+
+// NW: the most waves of the launch (8 up to K = 4096: a quarter more registers and LDS a wave)
+template <int T, int PER, int NW>
+__global__ __launch_bounds__(64 * NW) void gemv_kernel(GemvArgs a) {
+  __shared__ __align__(16) char dig[NW * kDigitBytes];
+  __shared__ float red[NW * kTileRows * T];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int N = a.N0 + a.N1 + a.N2;
+  const int n0 = blockIdx.x * kTileRows * T;
+  // each thread's first row's residual, loaded before anything waits
+  const int nr = n0 + threadIdx.x;
+  const float res = a.resid && threadIdx.x < kTileRows * T && nr < N ? a.resid[nr] : 0.0f;
+  gemv_part<T, PER>(a.x, a.K, a.sign, a.scales, n0, N, wave, lane, dig + wave * kDigitBytes, red);
+  __syncthreads();
+  for (int r = threadIdx.x; r < kTileRows * T; r += blockDim.x) {
+    const int n = n0 + r;
+    if (n >= N) return;
+    const float tot = gemv_row<T, NW>(red, r, blockDim.x >> 6);
+    const float y = a.resid ? tot + (r == (int)threadIdx.x ? res : a.resid[n]) : tot;
+    if (n < a.N0) a.out0[n] = y;
+    else if (n < a.N0 + a.N1) a.out1[n - a.N0] = y;
+    else a.out2[n - a.N0 - a.N1] = y;
+  }
+}
+
+template <int T>
+static void launch_gemv_t(const GemvArgs& a, int N, hipStream_t st) {
+  const dim3 g((N + kTileRows * T - 1) / (kTileRows * T)), b(64 * gemv_split(a.K).waves);
+  const GemvSplit sp = gemv_split(a.K);
+  if (sp.per == 1 && sp.waves <= 8) hipLaunchKernelGGL((gemv_kernel<T, 1, 8>), g, b, 0, st, a);
+  else if (sp.per == 1) hipLaunchKernelGGL((gemv_kernel<T, 1, 16>), g, b, 0, st, a);
+  else if (sp.per == 2) hipLaunchKernelGGL((gemv_kernel<T, 2, 16>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((gemv_kernel<T, 0, 16>), g, b, 0, st, a);
 }
 
 hipError_t launch_gemv(const GemvArgs& a, hipStream_t st) {
   const int N = a.N0 + a.N1 + a.N2;
   if (N <= 0) return hipSuccess;
-  const int waves = (N + kGemvRW - 1) / kGemvRW;
-  const dim3 g((waves + kGemvWaves - 1) / kGemvWaves);
-  if (a.K <= kLutMaxK) {
-    const size_t lds = gemv_lut_bytes(a.K);
-    const hipError_t e = gemv_allow_lds((const void*)gemv_kernel<kXLut>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(gemv_kernel<kXLut>, g, dim3(kGemvThreads), lds, st, a);
-  } else if (a.K <= kGemvLdsMaxK) {
-    const size_t lds = (size_t)(a.K / 32) * kXPad * sizeof(float);
-    hipLaunchKernelGGL(gemv_kernel<kXLds>, g, dim3(kGemvThreads), lds, st, a);
-  } else {
-    hipLaunchKernelGGL(gemv_kernel<kXGlobal>, g, dim3(kGemvThreads), 0, st, a);
-  }
+  // One tile a workgroup spreads few rows over the most CUs (4096 rows: 3.3 us against 3.7 with
+  // two). From 512 tiles, two: x is converted half as often (24576 x 4096: 6.8 us against 8.2 with
+  // one, 7.2 to 8.0 with three to six; 768 tiles of 2048 weights, 3.7 and 3.8, do not care).
+  const int tiles = (N + kTileRows - 1) / kTileRows;
+  if (tiles <= 512) launch_gemv_t<1>(a, N, st);
+  else launch_gemv_t<2>(a, N, st);
   return hipGetLastError();
 }
 
 // ---- fused decode qkv projection + prologue ---------------------------------------------------
-// RPW rows a workgroup (RPW / kGemvRW waves): 32 (16 waves), or 24 (12 waves) when 32-row
-// workgroups would leave CUs idle (the 8B shape: 256 workgroups of 24 rows instead of 192 of 32,
-// 5.27 -> 5.19 us; the table reads are VALU-bound, so the rows a CU holds set that phase). 192 of
-// 32 rows measured 6.7 us against 384 of 16 rows, two on half the CUs (7.3 us), or 96 of 64 (7.5).
 // s_waitcnt vmcnt(0) with expcnt and lgkmcnt left alone (gfx9 encoding: vmcnt bits 3:0 and 15:14,
 // expcnt 6:4, lgkmcnt 11:8)
 constexpr int kWaitVm0 = 0x0F70;
-template <int RPW>
-constexpr int qkv_threads() { return 64 * RPW / kGemvRW; }
-typedef float floatx4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 size_t qkv_proj_raw_floats(int heads, int D) { return (size_t)heads * D; }
 
-// Workgroup v owns rows [v RPW, v RPW + RPW) of the [Q heads | K heads | V heads] x D output.
-// The workgroup holding a head's last row finishes that head: its rows of the head stay in LDS,
-// its rows of the next head (RPW < D: a workgroup can straddle two heads) and every other
-// workgroup's rows go into the gather buffer. The finisher's first wave polls the head's earlier
-// rows until none holds the empty marker (the data is the completion signal: no ticket, no store
-// acknowledgement to wait for) while its sibling waves finish their rows, and meets them at the
-// barrier only after the poll (5.05 -> 4.85 us at the 8B shape); it then writes the marker back
+// Workgroup v owns rows [v RPW, v RPW + RPW) of the [Q heads | K heads | V heads] x D output (RPW
+// divides D, so they are one head's). The workgroup holding a head's last rows finishes that head:
+// its rows stay in LDS, every other workgroup's go into the gather buffer. The finisher's first
+// wave polls the head's earlier rows until none holds the empty marker (the data is the completion
+// signal: no ticket, no store acknowledgement to wait for); it then writes the marker back
 // (written through: the next launch's workgroups may run on another XCD), normalizes, ropes and
 // stores the row with the prologue's arithmetic (bg_qkrow.h: bit-identical to bg_gemv_split
 // followed by bg_qkv_prologue). The rows a finisher waits on belong to lower workgroup indices,
@@ -349,15 +373,16 @@ size_t qkv_proj_raw_floats(int heads, int D) { return (size_t)heads * D; }
 // gives up stores NaN and raises the cache's error word). When the grid is a multiple of 8 and
 // every eighth of the rows is whole heads, blockIdx 8m + x is workgroup v = x (grid / 8) + m, so
 // with round-robin placement each XCD holds a run of whole heads and the raw rows stay in its L2.
-template <int D, int DT, int XM, int RPW>
-__global__ __launch_bounds__(qkv_threads<RPW>()) void qkv_proj_kernel(LayerView L, QkvProjArgs a) {
-  constexpr int NT = qkv_threads<RPW>();
+template <int D, int DT, int T, int PER, int NW>
+__global__ __launch_bounds__(64 * NW) void qkv_proj_kernel(LayerView L, QkvProjArgs a) {
+  constexpr int RPW = kTileRows * T;
   constexpr int LPR = D / 4;  // lanes per row in the epilogue
   constexpr int kSC1 = 16;    // cache policy sc1: agent scope
-  extern __shared__ __align__(16) float xs[];
+  static_assert(RPW <= 64 && D % RPW == 0, "rows of a workgroup");
+  __shared__ __align__(16) char dig[NW * kDigitBytes];
+  __shared__ float red[NW * RPW];
   __shared__ __align__(16) float rrow[D];
   __shared__ __align__(16) float own[RPW];
-  // wave-uniform (scalar): the finisher's waves take different branches around one barrier
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int KV = L.kv_heads;
   const int nq = a.H * D;
@@ -366,55 +391,29 @@ __global__ __launch_bounds__(qkv_threads<RPW>()) void qkv_proj_kernel(LayerView 
   const bool grouped = (nwg & 7) == 0 && ((nwg >> 3) * RPW) % D == 0;
   const int v = grouped ? (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int r0 = v * RPW;
-  const int head = r0 / D;  // of the first row; 0 .. H-1: Q heads, then K heads, then V heads
-  const int hend = (head + 1) * D;
-  const bool finisher = r0 + RPW >= hend;  // holds the head's last row
-  const int own0 = r0 - head * D;          // the finisher's first dim of the head
+  const int head = r0 / D;  // 0 .. H-1: Q heads, then K heads, then V heads
+  const bool finisher = r0 + RPW == (head + 1) * D;  // holds the head's last rows
+  const int own0 = r0 - head * D;                    // the workgroup's first dim of the head
   // raw rows stay in the XCD's L2 when every workgroup of the head shares it
   const bool local = grouped && a.n_xcd == 8;
-  {
-    const int n0 = r0 + wave * kGemvRW;
-    GemvTile<kGemvRW> A;
-    float tot[kGemvRW];
-    if constexpr (XM == kXLut) {
-      // x first, then both tiles' weights (branch-free), so the table is built under their latency
-      LutX<NT> X;
-      gemv_lut_load<NT>(a.x, a.K, X);
-      GemvTile<kGemvRW> B;
-      gemv_load_w<kGemvRW, true>(A, a.K >> 5, a.K >> 7, a.sign, a.scales, n0, N, 0, lane);
-      gemv_load_w<kGemvRW, true>(B, a.K >> 5, a.K >> 7, a.sign, a.scales, n0, N, 1, lane);
-      gemv_lut_write<NT>(X, xs, a.K);
-      gemv_lut_rows<kGemvRW>(A, B, xs, a.K >> 5, lane, tot);
-    } else {
-      gemv_load_w<kGemvRW>(A, a.K >> 5, a.K >> 7, a.sign, a.scales, n0, N, 0, lane);
-      if constexpr (XM == kXLds) gemv_stage_x(a.x, xs, a.K);
-      gemv_rows<kGemvRW, XM, false>(A, a.x, xs, a.K, a.sign, a.scales, n0, N, lane, tot);
-    }
-#pragma unroll
-    for (int r = 0; r < kGemvRW; r++) {
-      const int n = n0 + r;
-      if (lane != r) continue;
-      if (finisher && n < hend) {
-        own[n - r0] = tot[r];
-      } else if (local) {
-        a.raw[n] = tot[r];  // into the XCD's L2
-      } else {
-        st_coherent(a.raw + n, tot[r]);
-      }
-    }
+  gemv_part<T, PER>(a.x, a.K, a.sign, a.scales, r0, N, wave, lane, dig + wave * kDigitBytes, red);
+  __syncthreads();
+  if (wave != 0) return;
+  // the first wave: one row a lane
+  if (lane < RPW) {
+    const float tot = gemv_row<T, NW>(red, lane, blockDim.x >> 6);
+    if (finisher) own[lane] = tot;
+    else if (local) a.raw[r0 + lane] = tot;  // into the XCD's L2
+    else st_coherent(a.raw + r0 + lane, tot);
   }
   if (!finisher) return;
-  if (wave != 0) {
-    __syncthreads();  // publishes this wave's rows in own[]; wave 0 polls before it meets them
-    return;
-  }
 
   // ---- the finishing part of the head: one wave, 4 dims a lane (D=128: both halves of the
   // wave hold the row; the lower one stores) ----
   const int c = lane % LPR;
   const bool writer = lane < LPR;
   const bool isq = head < a.H, isk = !isq && head < a.H + KV;
-  const bool mine = 4 * c >= own0;  // own0 is a multiple of 8
+  const bool mine = 4 * c >= own0;  // own0 is a multiple of 16
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.raw + (size_t)head * D, (short)0,
                                                                       D * 4, 0x00020000);
   // the row's gamma and rope tables are loaded before the wait, so the epilogue starts on arrival
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(qkv_threads<RPW>()) void qkv_proj_kernel(LayerView 
   float g[4] = {1.0f, 1.0f, 1.0f, 1.0f}, cs[4], sn[4];
   if (isq || isk) load4((isq ? a.q_gamma : a.k_gamma) + 4 * c, g);
   if (rope) row_tables(a.cos_tab, a.sin_tab, a.pos, a.rot_dim, c, cs, sn);
-  // the other workgroups' rows are polled before the barrier, under the sibling waves' rows
+  // the other workgroups' rows
   float x[4];
   bool gave_up = false;
   if (!mine) {
@@ -442,7 +441,9 @@ __global__ __launch_bounds__(qkv_threads<RPW>()) void qkv_proj_kernel(LayerView 
     }
     gave_up = missing;
   }
-  __syncthreads();  // the sibling waves' rows in own[]
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // own[], written by this wave
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (mine) {
 #pragma unroll
     for (int e = 0; e < 4; e++) x[e] = own[4 * c + e - own0];
@@ -489,41 +490,27 @@ __global__ __launch_bounds__(qkv_threads<RPW>()) void qkv_proj_kernel(LayerView 
   if (gave_up && lane == 0) __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-template <int D, int DT, int XM, int RPW>
-static hipError_t launch_qkv_proj_k(const LayerView& L, const QkvProjArgs& a, dim3 g, size_t lds, hipStream_t st) {
-  if constexpr (XM == kXLut) {
-    const hipError_t e = gemv_allow_lds((const void*)qkv_proj_kernel<D, DT, XM, RPW>, lds);
-    if (e != hipSuccess) return e;
+template <int D, int T, int PER, int NW>
+static hipError_t launch_qkv_proj_t(const LayerView& L, const QkvProjArgs& a, hipStream_t st) {
+  const dim3 g((a.H + 2 * L.kv_heads) * D / (kTileRows * T)), b(64 * gemv_split(a.K).waves);
+  switch (L.dtype) {
+    case KV_F32: hipLaunchKernelGGL((qkv_proj_kernel<D, KV_F32, T, PER, NW>), g, b, 0, st, L, a); break;
+    case KV_F16: hipLaunchKernelGGL((qkv_proj_kernel<D, KV_F16, T, PER, NW>), g, b, 0, st, L, a); break;
+    default: hipLaunchKernelGGL((qkv_proj_kernel<D, KV_Q8, T, PER, NW>), g, b, 0, st, L, a);
   }
-  hipLaunchKernelGGL((qkv_proj_kernel<D, DT, XM, RPW>), g, dim3(qkv_threads<RPW>()), lds, st, L, a);
   return hipGetLastError();
 }
 
-template <int D, int XM, int RPW>
-static hipError_t launch_qkv_proj_d(const LayerView& L, const QkvProjArgs& a, dim3 g, size_t lds, hipStream_t st) {
-  switch (L.dtype) {
-    case KV_F32: return launch_qkv_proj_k<D, KV_F32, XM, RPW>(L, a, g, lds, st);
-    case KV_F16: return launch_qkv_proj_k<D, KV_F16, XM, RPW>(L, a, g, lds, st);
-    default: return launch_qkv_proj_k<D, KV_Q8, XM, RPW>(L, a, g, lds, st);
-  }
-}
-
-template <int D, int RPW>
-static hipError_t launch_qkv_proj_x(const LayerView& L, const QkvProjArgs& a, dim3 g, hipStream_t st) {
-  if (a.K <= kLutMaxK) return launch_qkv_proj_d<D, kXLut, RPW>(L, a, g, gemv_lut_bytes(a.K), st);
-  if (a.K <= kGemvLdsMaxK)
-    return launch_qkv_proj_d<D, kXLds, RPW>(L, a, g, (size_t)(a.K / 32) * kXPad * sizeof(float), st);
-  return launch_qkv_proj_d<D, kXGlobal, RPW>(L, a, g, 0, st);
+// 32 rows a workgroup: 192 workgroups for the 8B shape, 4.82 us; 16 rows (384) 5.0, 64 (96) 5.7
+template <int D>
+static hipError_t launch_qkv_proj_d(const LayerView& L, const QkvProjArgs& a, hipStream_t st) {
+  const GemvSplit sp = gemv_split(a.K);
+  if (sp.per == 1 && sp.waves <= 8) return launch_qkv_proj_t<D, 2, 1, 8>(L, a, st);
+  return sp.per == 1 ? launch_qkv_proj_t<D, 2, 1, 16>(L, a, st) : launch_qkv_proj_t<D, 2, 0, 16>(L, a, st);
 }
 
 hipError_t launch_qkv_proj(const LayerView& L, const QkvProjArgs& a, hipStream_t st) {
-  const int N = (a.H + 2 * L.kv_heads) * L.D;
-  // 24-row workgroups (D = 128) when 32-row ones would leave CUs idle and the rows fall into 8
-  // runs of whole heads (one an XCD)
-  if (L.D == 128 && N / 32 < a.num_cus && N % (24 * 8) == 0 && (N / 8) % 128 == 0)
-    return launch_qkv_proj_x<128, 24>(L, a, dim3(N / 24), st);
-  const dim3 g(N / 32);
-  return L.D == 128 ? launch_qkv_proj_x<128, 32>(L, a, g, st) : launch_qkv_proj_x<256, 32>(L, a, g, st);
+  return L.D == 128 ? launch_qkv_proj_d<128>(L, a, st) : launch_qkv_proj_d<256>(L, a, st);
 }
 
 }  // namespace bg
