@@ -39,7 +39,12 @@ struct bg_kv_cache {
   size_t ws_counters = 0;
   // f16 copy of one q8 layer's attended slots for long prefills (K then V, cap_copy slots each)
   void* pf16 = nullptr;
-  float* pf_ml = nullptr;  // split-K prefill (m, l), bg::prefill_split_ml_bytes() once allocated
+  // split-K prefill: partials (a larger buffer replaces a smaller one, which is kept until destroy
+  // for the launches captured with it) and their (m, l), bg::kPfSplitMlBytes once allocated
+  float* pf_o = nullptr;
+  size_t pf_floats = 0;
+  float* pf_ml = nullptr;
+  std::vector<float*> retired_pf;
   // workspaces replaced by a larger one, kept until destroy: launches captured in a graph before
   // the growth still use them (and find their slots holding the empty marker)
   std::vector<std::pair<float*, size_t>> retired_ws;
@@ -139,11 +144,10 @@ int addressable(const bg_kv_cache* c) { return c->roll ? c->max_seq : c->capacit
 // the array's name to a kernel (on the host it is a stand-in, not a device address): the device
 // address comes from hipGetSymbolAddress, once per device, and only that pointer is used.
 // Between launches every slot holds the decode kernel's empty marker; the set-up fills it once.
-// Layout: the first kScratchBytes hold split partials (decode, split-K prefill) and the empty
-// marker between launches; the kScratchMlBytes after them hold a split-K prefill's (m, l) values.
+// Layout: the first kScratchBytes hold the decode's split partials and the empty marker between
+// launches; a split-K prefill's partials and their (m, l) values follow.
 constexpr size_t kScratchBytes = (size_t)8 << 20;     // 8 MiB per GPU
-constexpr size_t kScratchMlBytes = (size_t)256 << 10;  // 256 KiB
-__device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchMlBytes];
+__device__ __align__(256) unsigned char scratch[kScratchBytes + bg::kPfSplitBytes + bg::kPfSplitMlBytes];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
@@ -481,7 +485,9 @@ int32_t bg_kv_destroy(bg_kv_cache* c) {
   if (c->ws) (void)hipFree(c->ws);
   if (c->ws_count) (void)hipFree(c->ws_count);
   if (c->pf16) (void)hipFree(c->pf16);
+  if (c->pf_o) (void)hipFree(c->pf_o);
   if (c->pf_ml) (void)hipFree(c->pf_ml);
+  for (float* r : c->retired_pf) (void)hipFree(r);
   for (const auto& r : c->retired_ws) (void)hipFree(r.first);
   for (unsigned* r : c->retired_count) (void)hipFree(r);
   delete c;
@@ -637,8 +643,8 @@ int32_t bg_qkv_prologue(bg_kv_cache* c, int32_t layer, const float* q, int32_t q
   return e == hipSuccess ? BG_OK : hip_fail(e, "prologue launch");
 }
 
-// The attention workspace: decode split partials, f32 split partials or split-K prefill partials
-// (each launch uses one kind; every slot holds the empty marker between launches). Grows to at
+// The attention workspace: decode or f32 split partials (each launch uses one kind; every slot
+// holds the empty marker between launches). Grows to at
 // least `need` floats and `counters` counters, keeping the larger of old and new.
 static int32_t ensure_workspace_floats(bg_kv_cache* c, size_t need, size_t counters) {
   if (need < c->ws_floats) need = c->ws_floats;
@@ -674,16 +680,31 @@ static int32_t ensure_workspace_floats(bg_kv_cache* c, size_t need, size_t count
   return BG_OK;
 }
 
-// split-K prefill: partials in the workspace, (m, l) in a buffer of their own
-static int32_t ensure_prefill_split(bg_kv_cache* c, size_t floats) {
-  int32_t rc = ensure_workspace_floats(c, floats, 0);
-  if (rc != BG_OK || c->pf_ml) return rc;
-  hipError_t e = hipMalloc((void**)&c->pf_ml, bg::prefill_split_ml_bytes());
+// Split-K prefill: buffers for `floats` floats of partials and their (m, l). False when they cannot
+// be had (out of memory, or the stream is being captured): the launch then scans whole key ranges,
+// which needs none.
+static bool ensure_prefill_split(bg_kv_cache* c, size_t floats, hipStream_t st) {
+  if (floats <= c->pf_floats && c->pf_ml) return true;
+  if (capturing(st)) return false;
+  if (floats < 2 * c->pf_floats) floats = 2 * c->pf_floats;  // few buffers are ever retired
+  if (floats > bg::kPfSplitBytes / sizeof(float)) floats = bg::kPfSplitBytes / sizeof(float);
+  float* o = nullptr;
+  float* ml = nullptr;
+  hipError_t e = hipSuccess;
+  if (floats > c->pf_floats) e = hipMalloc((void**)&o, floats * sizeof(float));
+  if (e == hipSuccess && !c->pf_ml) e = hipMalloc((void**)&ml, bg::kPfSplitMlBytes);
   if (e != hipSuccess) {
-    c->pf_ml = nullptr;
-    return hip_fail(e, "split prefill (m, l) allocation");
+    (void)hipGetLastError();
+    if (o) (void)hipFree(o);
+    return false;
   }
-  return BG_OK;
+  if (o) {
+    if (c->pf_o) c->retired_pf.push_back(c->pf_o);
+    c->pf_o = o;
+    c->pf_floats = floats;
+  }
+  if (ml) c->pf_ml = ml;
+  return true;
 }
 
 static int32_t ensure_workspace(bg_kv_cache* c, int S, int H) {
@@ -723,8 +744,10 @@ int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
       int32_t rc = ensure_prefill_copy(c);
       if (rc != BG_OK) return rc;
     }
-    const size_t pf = bg::prefill_workspace_floats_max(view(c, 0), S, H, c->num_cus);
-    return pf > 0 ? ensure_prefill_split(c, pf) : BG_OK;
+    if (bg::prefill_can_split(view(c, 0), S, H, c->num_cus) &&
+        !ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
+      return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
+    return BG_OK;
   }
   if (!bg::decode_supported(view(c, 0), S, H) && !bg::f32_split_supported(view(c, 0), S, H)) return BG_OK;
   return ensure_workspace(c, S, H);
@@ -764,7 +787,9 @@ static bg::AttnArgs attention_args(bg_kv_cache* c, const float* q, int32_t S, in
   a.out = out;
   a.ws_o = nullptr;
   a.ws_ml = nullptr;
+  a.pf_o = nullptr;
   a.pf_ml = nullptr;
+  a.pf_floats = 0;
   a.ws_count = nullptr;
   a.ws_floats = 0;
   a.num_cus = c->num_cus;
@@ -804,12 +829,10 @@ int32_t bg_attention(bg_kv_cache* c, int32_t layer, const float* q, int32_t S, i
     e = bg::launch_attention_decode(L, a, st);
   } else if (bg::prefill_supported(L, S, H)) {
     const size_t pf = bg::prefill_workspace_floats(L, S, H, pos_base, c->num_cus);
-    if (pf > 0) {
-      int32_t rc = ensure_prefill_split(c, pf);
-      if (rc != BG_OK) return rc;
-      a.ws_o = c->ws;
-      a.ws_floats = c->ws_floats;
+    if (pf > 0 && ensure_prefill_split(c, pf, st)) {
+      a.pf_o = c->pf_o;
       a.pf_ml = c->pf_ml;
+      a.pf_floats = c->pf_floats;
     }
     if (bg::prefill_wants_f16_copy(L, S, H)) {
       // dequantize the attended slots once, then run the f16 path on the copy
@@ -884,12 +907,10 @@ int32_t bg_attention_noalloc(bg_kv_cache* c, int32_t layer, const float* q, int3
     e = bg::launch_attention_decode(L, a, st);
   } else if (bg::prefill_supported(L, S, H)) {
     // a q8 cache is staged in-kernel (no f16 copy): the same values, so the same results; a
-    // split-K prefill keeps its partials in the scratch (the split plan caps them below it)
-    if (bg::prefill_split_ml_bytes() > kScratchMlBytes)
-      return fail(BG_E_UNSUPPORTED, "bg_attention_noalloc: the scratch's (m, l) area is smaller than a split prefill needs");
-    a.ws_o = (float*)ptr;
-    a.ws_floats = kScratchBytes / sizeof(float);
-    a.pf_ml = (float*)((char*)ptr + kScratchBytes);
+    // split-K prefill keeps its partials in the scratch, which holds every plan's
+    a.pf_o = (float*)((char*)ptr + kScratchBytes);
+    a.pf_floats = bg::kPfSplitBytes / sizeof(float);
+    a.pf_ml = (float*)((char*)ptr + kScratchBytes + bg::kPfSplitBytes);
     e = bg::launch_attention_prefill(L, a, st);
   } else {
     return fail(BG_E_UNSUPPORTED, "bg_attention_noalloc: no kernel for S %d, heads %d", S, H);

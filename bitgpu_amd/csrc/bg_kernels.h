@@ -96,9 +96,9 @@ struct AttnArgs {
   float* out;
   // split-K workspace
   float* ws_o; float* ws_ml; unsigned* ws_count; size_t ws_floats;
-  // split-K prefill: (m, l) of the partials, prefill_split_ml_bytes() long (outside ws_o, whose
-  // slots hold the empty marker between launches)
-  float* pf_ml;
+  // split-K prefill: the partials (pf_floats long) and their (m, l), kPfSplitMlBytes long; a launch
+  // whose plan needs more than is there scans whole key ranges
+  float* pf_o; float* pf_ml; size_t pf_floats;
   int num_cus;
   // decode merge: host-visible error word, poll bound (0: default) and a test hook that makes
   // one split store no partial (-1: none)
@@ -148,13 +148,16 @@ bool prefill_supported(const LayerView& L, int S, int H);
 // f16 copy of the attended slots
 bool prefill_wants_f16_copy(const LayerView& L, int S, int H);
 // "not written yet" marker of a split partial slot: a quiet NaN with a payload arithmetic on
-// finite inputs never produces. The decode and split-K prefill kernels share the workspace and
-// both leave every slot they use holding it.
+// finite inputs never produces. The decode kernel leaves every slot it uses holding it.
 constexpr uint32_t kWorkspaceEmpty = 0x7FF1DE5Au;
-// workspace floats a prefill launch's split-K partials use at pos_base (0: the launch does not
-// split); the most any pos_base can use for S rows of H heads is prefill_workspace_floats_max
+// A split-K prefill plan's largest partials: 512 workgroups of 64 KB at head_dim 128, 256 of 128 KB
+// at 256 (one round of a 256-CU GPU), and 512 x 4 waves x 64 lanes of (m, l).
+constexpr size_t kPfSplitBytes = (size_t)32 << 20;
+constexpr size_t kPfSplitMlBytes = (size_t)1 << 20;
+constexpr int kPfMaxParts = 512;
+// floats of the partials a prefill launch uses at pos_base (0: the launch does not split); whether
+// S rows of H heads can split at any pos_base (the partials are then at most kPfSplitBytes)
 size_t prefill_workspace_floats(const LayerView& L, int S, int H, int pos_base, int num_cus);
-size_t prefill_workspace_floats_max(const LayerView& L, int S, int H, int num_cus);
-size_t prefill_split_ml_bytes();
+bool prefill_can_split(const LayerView& L, int S, int H, int num_cus);
 
 }  // namespace bg

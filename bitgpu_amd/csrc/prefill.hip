@@ -81,7 +81,7 @@ struct PrefillParams {
   // scanned by its own workgroup, which leaves its partial in pws for prefill_merge_kernel
   int n_parts, part_steps;
   int split_waves;   // waves whose rows can be valid (fewer when the grid has fewer rows than 128)
-  float4* pws;       // [item][part][split_waves][4 * D/32][64] float4: o slots (empty marker between launches)
+  float4* pws;       // [item][part][split_waves][4 * D/32][64] float4: o slots
   float2* pml;       // [item][part][split_waves][64] (m, l) of each lane's row
 };
 
@@ -340,14 +340,15 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
   // the CUs hold at once (mirror) pairs them: workgroup b < n/2 takes item b, the rest the mirrors
   // n-1-(b-n/2), so that each CU holds one heavy and one light item and every CU scans about the
   // same number of keys. A larger grid runs heaviest first, balanced by the dispatcher.
-  // Split-K (a grid far smaller than the GPU): workgroup b scans part b % n_parts of item
-  // b / n_parts.
+  // Split-K (a grid that leaves CUs idle): the kv head is the fastest index, as in the other
+  // grids, so with 8 (or 4) kv heads the workgroups of one share an XCD's L2, then the part.
   const int bid = blockIdx.x;
   const int n_items = p.n_qblocks * KV;
   const int half = (n_items + 1) / 2;
   const bool split = p.n_parts > 1;
-  const int part = split ? bid % p.n_parts : 0;
-  const int item = split ? bid / p.n_parts : !p.mirror || bid < half ? bid : n_items - 1 - (bid - half);
+  const int part = split ? bid / KV % p.n_parts : 0;
+  const int item = split ? bid / (KV * p.n_parts) * KV + bid % KV
+                         : !p.mirror || bid < half ? bid : n_items - 1 - (bid - half);
   const int kvh = item % KV;
   const int qb = p.n_qblocks - 1 - item / KV;
   const int s0 = qb * p.QB;
@@ -795,9 +796,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
 
 // Split-K merge: workgroup (item, wave, o slot) combines that slot of the wave's 32 rows over the
 // parts by log-sum-exp, applies the gate (gate_sigmoid.wgsl:13 form) and stores the output
-// float4s; the four 64-lane groups take every fourth part and meet through LDS. Every o slot it
-// read gets the empty marker back, so the workspace the decode kernel shares keeps its invariant
-// (the (m, l) values live outside that workspace and are only read).
+// float4s; the four 64-lane groups take every fourth part and meet through LDS. It only reads the
+// partials (a buffer of their own: the decode kernel's workspace, whose slots must hold the empty
+// marker between launches, would have to be written back here, as many bytes as the read).
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
   constexpr int KT = PfCfg<D>::KT, ND = D / 32, NSL = 4 * ND;
@@ -845,8 +846,6 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
   red_m[grp][lane] = mx;
   __syncthreads();
   const float M = fmaxf(fmaxf(red_m[0][lane], red_m[1][lane]), fmaxf(red_m[2][lane], red_m[3][lane]));
-  const float em = __uint_as_float(kWorkspaceEmpty);
-  const float4 empty = make_float4(em, em, em, em);
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   float lt = 0.0f;
   if (batch) {
@@ -854,14 +853,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     for (int j = 0; j < PB; j++) {
       const int q = grp + 4 * j;
       if (q < np) {
-        const size_t pi = pi0 + q * pstride;
         const float w = __builtin_amdgcn_exp2f(mlb[j].x - M);
         acc.x += vb[j].x * w;
         acc.y += vb[j].y * w;
         acc.z += vb[j].z * w;
         acc.w += vb[j].w * w;
         lt += mlb[j].y * w;
-        p.pws[(pi * NSL + sl) * 64 + lane] = empty;
       }
     }
   }
@@ -869,14 +866,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     const size_t pi = pi0 + q * pstride;
     const float2 ml = p.pml[pi * 64 + lane];
     const float w = __builtin_amdgcn_exp2f(ml.x - M);
-    float4* slot = p.pws + (pi * NSL + sl) * 64 + lane;
-    const float4 v = *slot;
+    const float4 v = p.pws[(pi * NSL + sl) * 64 + lane];
     acc.x += v.x * w;
     acc.y += v.y * w;
     acc.z += v.z * w;
     acc.w += v.w * w;
     lt += ml.y * w;
-    *slot = empty;
   }
   red_o[grp][lane] = acc;
   red_l[grp][lane] = lt;
@@ -927,15 +922,17 @@ bool prefill_wants_f16_copy(const LayerView& L, int S, int H) {
 // dispatcher.
 static bool pf_mirror(const LayerView& L, int n_items, int num_cus) { return L.D == 128 && n_items <= 2 * num_cus; }
 
-// Split-K plan of a prefill launch. A grid of (query block, kv head) items far smaller than the
-// GPU (short prompts after a long context, speculative verify with many heads per kv head) leaves
-// most CUs idle while each workgroup scans the whole key range; such a grid is split into parts
-// of at least kPfMinPartSteps steps, up to a full GPU's worth of workgroups, with all partials
-// within kPfSplitMaxBytes (the allocation-free entry point's scratch holds them too, so both
-// entry points make the same split and return the same results).
-constexpr size_t kPfSplitMaxBytes = (size_t)8 << 20;
+// Split-K plan of a prefill launch. A grid of (query block, kv head) items that leaves CUs idle
+// (a user turn or verify after a long context) splits every item's key range into parts of at
+// least kPfMinPartSteps steps, at most one round of workgroups. The part count is the cheapest by
+// a cost model in microseconds, its constants measured: a step takes about 1 us of a CU, 2.1 us
+// where a D=128 CU runs two workgroups; a part's partial (32 KB a wave at D=256, 16 KB at D=128)
+// is written and read at about 4.5 TB/s, and the merge kernel adds about 6 us. So a short prompt stays whole
+// (S=500: 14.8 us, 31 split in two) and a turn of 333 tokens after 12,000 takes five parts (184 ->
+// 107 us; two 127, three 135), 300 after 3,000 at D=256 four (129 -> 68 us; two 86, eight 83).
+// Both entry points use the same plan (the allocation-free one's scratch holds every plan's
+// partials), so their results are the same.
 constexpr int kPfMinPartSteps = 4;
-constexpr size_t kPfSplitMlBytes = (size_t)256 << 10;  // (m, l) of the split partials
 struct PfSplitPlan {
   int n_parts, part_steps, waves;
   size_t floats;
@@ -948,23 +945,28 @@ static PfSplitPlan pf_split_plan(const LayerView& L, int S, int H, int pos_base,
   const int per_cu = L.D == 128 ? 2 : 1;  // workgroups a CU holds
   const long slots = (L.ring.roll && L.ring.head != 0) ? (long)L.max_seq : (long)pos_base + S;
   const int steps_max = (int)((slots + KT - 1) / KT);
-  if (2 * n_items > per_cu * num_cus) return r;
   // partials only for the waves holding rows: (query, head) rows of a block, 32 a wave
   const int waves = std::min(4, (std::min(QB, S) * G + 31) / 32);
   const size_t part_bytes = (size_t)waves * 4 * (L.D / 32) * 64 * sizeof(float4);
   const size_t ml_bytes = (size_t)waves * 64 * sizeof(float2);
-  int P = per_cu * num_cus / n_items;
-  P = std::min(P, steps_max / kPfMinPartSteps);
-  P = std::min(P, (int)(kPfSplitMaxBytes / (part_bytes * n_items)));
+  int P = std::min(std::min(per_cu * num_cus / n_items, steps_max / kPfMinPartSteps), kPfMaxParts);
+  P = std::min(P, (int)(kPfSplitBytes / (part_bytes * n_items)));
   P = std::min(P, (int)(kPfSplitMlBytes / (ml_bytes * n_items)));
-  if (P < 2) return r;
-  const int ps = (steps_max + P - 1) / P;
-  const int np = (steps_max + ps - 1) / ps;
-  if (np < 2) return r;
-  r.n_parts = np;
-  r.part_steps = ps;
-  r.waves = waves;
-  r.floats = (size_t)n_items * np * part_bytes / sizeof(float);
+  const float us_part = 2.0f * part_bytes / 4.5e6f;
+  float best = steps_max * 1.0f;
+  if (n_items > num_cus) best *= 2.1f;
+  for (int np = 2; np <= P; np++) {
+    const int ps = (steps_max + np - 1) / np;
+    if ((steps_max + ps - 1) / ps != np) continue;  // the same split as fewer parts
+    const float t = ps * (n_items * np > num_cus ? 2.1f : 1.0f) + n_items * np * us_part + 6.0f;
+    if (t < best) {
+      best = t;
+      r.n_parts = np;
+      r.part_steps = ps;
+      r.waves = waves;
+      r.floats = (size_t)n_items * np * part_bytes / sizeof(float);
+    }
+  }
   return r;
 }
 
@@ -973,15 +975,11 @@ size_t prefill_workspace_floats(const LayerView& L, int S, int H, int pos_base, 
   return pf_split_plan(L, S, H, pos_base, num_cus).floats;
 }
 
-size_t prefill_split_ml_bytes() { return kPfSplitMlBytes; }
-
-size_t prefill_workspace_floats_max(const LayerView& L, int S, int H, int num_cus) {
-  if (!prefill_supported(L, S, H)) return 0;
+bool prefill_can_split(const LayerView& L, int S, int H, int num_cus) {
+  if (!prefill_supported(L, S, H)) return false;
   const int G = H / L.kv_heads, QB = 128 / G;
   const int n_items = (S + QB - 1) / QB * L.kv_heads;
-  const int per_cu = L.D == 128 ? 2 : 1;
-  if (2 * n_items > per_cu * num_cus) return 0;
-  return kPfSplitMaxBytes / sizeof(float);
+  return 2 * n_items <= (L.D == 128 ? 2 : 1) * num_cus;
 }
 
 template <int D, int DT, bool ROLL>
@@ -1016,12 +1014,12 @@ hipError_t launch_attention_prefill(const LayerView& L, const AttnArgs& a, hipSt
   p.pws = nullptr;
   p.pml = nullptr;
   const PfSplitPlan sp = pf_split_plan(L, a.S, a.H, a.pos_base, a.num_cus);
-  if (sp.n_parts > 1) {
-    if (!a.ws_o || !a.pf_ml || sp.floats > a.ws_floats) return hipErrorInvalidValue;  // the caller sizes them
+  // (without a buffer for the partials: a whole scan)
+  if (sp.n_parts > 1 && a.pf_o && a.pf_ml && sp.floats <= a.pf_floats) {
     p.n_parts = sp.n_parts;
     p.part_steps = sp.part_steps;
     p.split_waves = sp.waves;
-    p.pws = (float4*)a.ws_o;
+    p.pws = (float4*)a.pf_o;
     p.pml = (float2*)a.pf_ml;
     p.mirror = 0;
   }

@@ -18,9 +18,9 @@
  *     streams could overlap on the GPU and corrupt each other's partials.
  *   - Kernels never allocate. Host-side allocations happen only in bg_kv_create, bg_kv_grow,
  *     bg_attention_reserve, lazily on the first bg_attention that needs more workspace (split
- *     partials; a split-K prefill also a 256 KiB buffer of their (m, l) values) or, for a q8
- *     cache, the f16 copy a long prefill runs on, and in the snapshot transfers (a staging
- *     buffer kept by the cache, grown when a larger region is transferred).
+ *     partials, at most 33 MiB of them for a split-K prefill, which runs unsplit where they cannot
+ *     be had) or, for a q8 cache, the f16 copy a long prefill runs on, and in the snapshot
+ *     transfers (a staging buffer kept by the cache, grown when a larger region is transferred).
  *   - The decode kernel's split merge waits a bounded time for the partials of its own grid.
  *     If a wait gives up (the GPU shared with work that keeps the grid from running at once),
  *     that launch stores NaN and raises the cache's error word; the next bg_attention on the
@@ -249,13 +249,12 @@ int32_t bg_attention(bg_kv_cache* cache, int32_t layer, const float* q, int32_t 
 /* Allocation-free variant of bg_attention. No counterpart in the reference (WebGPU dispatches
  * never allocate per call); it is for callers that cannot call hipMalloc: code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation. Same arguments and results as
- * bg_attention, but it allocates nothing: the split partials of the decode kernel and of a
- * split-K prefill live in a file-scope device array of 8 MiB per GPU (plus 256 KiB for a split
- * prefill's (m, l) values; held until the process ends) instead of the cache's workspace (the
- * prefill splits only as far as 8 MiB of partials, for either entry point); a q8 prefill stages its tiles in-kernel instead of through the f16 copy
- * (the same values: identical output); an f32 cache runs the exact-f32 kernel of one wave per
- * (query, head), which keeps no partials (agrees with bg_attention to f32 rounding). A launch
- * whose partials would exceed the array is rejected with BG_E_INVALID before anything runs.
+ * bg_attention, but it allocates nothing: the split partials of the decode kernel (8 MiB per GPU)
+ * and of a split-K prefill (33 MiB, as much as any plan needs) live in a file-scope device array,
+ * held until the process ends, instead of the cache's workspace; a q8 prefill stages its tiles
+ * in-kernel instead of through the f16 copy (the same values: identical output); an f32 cache runs the exact-f32 kernel of one wave per
+ * (query, head), which keeps no partials (agrees with bg_attention to f32 rounding). A decode
+ * launch whose partials would exceed its 8 MiB is rejected with BG_E_INVALID before anything runs.
  * The first call on a device sets the array up (a fill kernel, synchronized) and must not be
  * under graph capture (BG_E_STATE). Every call on one GPU shares that GPU's array: calls that
  * overlap on the GPU (different streams, or different host threads) race and corrupt each

@@ -1,0 +1,49 @@
+"""GPU: a user turn of a few hundred tokens after a long context, whose prefill splits every
+item's key range over a full round of workgroups, against the oracle; the allocation-free entry
+point makes the same split (bit-identical); a capture without a reserved workspace scans whole
+key ranges instead. Tolerances as for every f16 / q8 attention (relative 2e-3)."""
+import numpy as np
+import pytest
+import torch
+
+from bitgpu_amd import engine as E
+from oracle import ref
+from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc, t
+from tests.test_gpu_split_prefill import _case, _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,H,KV,D,ctx,S,gate", [
+    ("q8", 32, 8, 128, 6001, 333, False),    # 88 items in five parts of 20 steps, the last shorter
+    ("f16", 16, 8, 128, 5000, 97, False),    # 16 items in many parts
+    ("q8", 24, 4, 256, 3001, 300, True),     # 60 items in four parts, gated
+    ("f16", 32, 8, 128, 2999, 250, False),   # 64 items
+])
+def test_turn_after_context(dev, dtype, H, KV, D, ctx, S, gate):
+    c, _, q, g = _case(dtype, H, KV, D, ctx + S, S, seed=ctx + S, gate=gate)
+    scale = 1.0 / np.sqrt(D)
+    out = run_attention(c, 0, q, ctx, scale=scale, gate=g)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    _check(out, ref.gated_attention(q, kk, vv, g, ctx) if gate else ref.attention(q, kk, vv, ctx, scale=scale))
+    assert np.array_equal(run_attention_noalloc(c, 0, q, ctx, scale=scale, gate=g), out)
+    c.close()
+
+
+def test_turn_captured_without_reserve(dev):
+    H, KV, D, ctx, S = 32, 8, 128, 5000, 200
+    c, _, q, _ = _case("f16", H, KV, D, ctx + S, S, seed=3, gate=False)
+    qt, out = t(q), torch.empty(S, H, D, device="cuda")
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        E.attention(c, 0, qt, S, H, ctx, out=out)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    want = ref.attention(q, kk, vv, ctx)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        _check(out.cpu().numpy(), want)
+    c.close()
