@@ -37,7 +37,7 @@ struct bg_kv_cache {
   size_t ws_floats = 0;
   unsigned* ws_count = nullptr;
   size_t ws_counters = 0;
-  // f16 copy of one q8 layer's attended slots for long prefills (K then V, cap_copy slots each)
+  // f16 copy of one q8 or sink-mode layer's attended slots for long prefills (K then, q8, V)
   void* pf16 = nullptr;
   // split-K prefill: partials (a larger buffer replaces a smaller one, which is kept until destroy
   // for the launches captured with it) and their (m, l), bg::kPfSplitMlBytes once allocated
@@ -724,7 +724,7 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
   if (c->pf16) (void)hipFree(c->pf16);
   c->pf16 = nullptr;
   c->pf16_cap = 0;
-  const size_t bytes = (size_t)2 * c->kv_heads * c->cap * c->D * sizeof(uint16_t);
+  const size_t bytes = (size_t)(c->dtype == BG_KV_Q8 ? 2 : 1) * c->kv_heads * c->cap * c->D * sizeof(uint16_t);
   hipError_t e = hipMalloc(&c->pf16, bytes);
   if (e == hipSuccess) e = hipMemset(c->pf16, 0, bytes);
   if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -790,6 +790,7 @@ static bg::AttnArgs attention_args(bg_kv_cache* c, const float* q, int32_t S, in
   a.pf_o = nullptr;
   a.pf_ml = nullptr;
   a.pf_floats = 0;
+  a.k_rotated = 0;
   a.ws_count = nullptr;
   a.ws_floats = 0;
   a.num_cus = c->num_cus;
@@ -834,19 +835,32 @@ int32_t bg_attention(bg_kv_cache* c, int32_t layer, const float* q, int32_t S, i
       a.pf_ml = c->pf_ml;
       a.pf_floats = c->pf_floats;
     }
-    if (bg::prefill_wants_f16_copy(L, S, H)) {
-      // dequantize the attended slots once, then run the f16 path on the copy
-      int32_t rc = ensure_prefill_copy(c);
-      if (rc != BG_OK) return rc;
-      int n = (pos_base + S + 63) & ~63;
+    bool copy = bg::prefill_wants_f16_copy(L, S, H);
+    if (copy && !(c->pf16 && c->pf16_cap == c->cap)) {
+      // sink mode can rotate at staging instead (the same values), where the copy cannot be had
+      if (c->roll && capturing(st)) {
+        copy = false;
+      } else {
+        int32_t rc = ensure_prefill_copy(c);
+        if (rc != BG_OK && !c->roll) return rc;
+        copy = rc == BG_OK;
+        if (!copy) (void)hipGetLastError();
+      }
+    }
+    if (copy) {
+      // convert the attended slots once, then run the f16 path on the copy; a ring whose origin has
+      // moved is scanned whole
+      int n = c->roll && c->head != 0 ? c->max_seq : pos_base + S;
+      n = (n + 63) & ~63;
       n = n < c->cap ? n : c->cap;
       LayerView F = L;
       F.k = c->pf16;
-      F.v = (uint16_t*)c->pf16 + (size_t)c->kv_heads * c->cap * c->D;
+      if (c->dtype == BG_KV_Q8) F.v = (uint16_t*)c->pf16 + (size_t)c->kv_heads * c->cap * c->D;
       F.ks = nullptr;
       F.vs = nullptr;
       F.dtype = bg::KV_F16;
-      e = bg::launch_kv_dequant_f16(L, n, F.k, F.v, st);
+      a.k_rotated = c->roll;
+      e = bg::launch_kv_prefill_copy(L, n, F.k, F.v, st);
       if (e == hipSuccess) e = bg::launch_attention_prefill(F, a, st);
     } else {
       e = bg::launch_attention_prefill(L, a, st);

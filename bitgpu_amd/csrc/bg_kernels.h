@@ -35,9 +35,10 @@ hipError_t launch_kv_write(const LayerView& L, int which, const float* src, int 
                            hipStream_t st);
 hipError_t launch_kv_export(const LayerView& L, int region, int base, int count, void* dst, hipStream_t st);
 hipError_t launch_kv_import(const LayerView& L, int region, int base, int count, const void* src, hipStream_t st);
-// q8 layer -> f16 copy of slots [0, n_slots) (n_slots a multiple of 32) laid out like an f16
-// cache of the same capacity, with the q8 prefill staging's exact values
-hipError_t launch_kv_dequant_f16(const LayerView& L, int n_slots, void* kdst, void* vdst, hipStream_t st);
+// f16 copy of slots [0, n_slots) (n_slots a multiple of 32) of a q8 or sink-mode layer, laid out
+// like an f16 cache of the same capacity, with the prefill staging's exact values: q8 dequantized,
+// sink-mode keys rotated at their slot's position. An f16 layer's V is not copied (vdst unused).
+hipError_t launch_kv_prefill_copy(const LayerView& L, int n_slots, void* kdst, void* vdst, hipStream_t st);
 
 // norm_rope.hip
 struct PrologueArgs {
@@ -99,6 +100,7 @@ struct AttnArgs {
   // split-K prefill: the partials (pf_floats long) and their (m, l), kPfSplitMlBytes long; a launch
   // whose plan needs more than is there scans whole key ranges
   float* pf_o; float* pf_ml; size_t pf_floats;
+  int k_rotated;   // prefill, sink mode: the layer's keys are already rotated (the f16 copy)
   int num_cus;
   // decode merge: host-visible error word, poll bound (0: default) and a test hook that makes
   // one split store no partial (-1: none)

@@ -92,38 +92,80 @@ hipError_t launch_kv_import(const LayerView& L, int region, int base, int count,
   return hipGetLastError();
 }
 
-// ---- q8 -> f16 copy of the attended slots, for a long prefill ---------------------------------
-// A q8 prefill stages (dequantizes) every K/V tile once per query block that attends it. For a
-// long prompt the attended slots are dequantized once here into an f16 copy laid out like an f16
-// cache (K row-major, V in 32-slot transposed tiles), and the prefill runs its direct-to-LDS f16
-// path on that copy. The values are exactly the ones the q8 staging produces: the code, biased
-// to u = code + 128, times s = scale * (1/127) in one f32 fma (u * s - 128 * s), then RNE to f16
-// (q8_stage_f16).
+// ---- f16 copy of the attended slots, for a long prefill ----------------------------------------
+// A prefill stages every K/V tile once per query block that attends it. Where staging computes
+// (q8: dequantize, sink mode: rotate the keys) and there are blocks enough, the attended slots are
+// converted once here into a copy laid out like an f16 cache (K row-major, V in 32-slot
+// transposed tiles), and the prefill copies its tiles from that straight into LDS. The values
+// are exactly the staging's: q8 the code, biased to u = code + 128, times s = scale * (1/127) in
+// one f32 fma (u * s - 128 * s); sink mode the pair (x, y) of dims (i, i + D/2) rotated at the
+// slot's position in f32, every product and sum rounded; then RNE to f16. Bound by memory: each
+// value read once and written once (4100 slots of 8 heads, f16 keys: 17 MB; 12,334 slots q8, K and
+// V: 78 MB in 15 us).
 
-template <int D>
-__global__ __launch_bounds__(256) void kv_dequant_kernel(LayerView L, int n_slots, __half* __restrict__ kdst,
-                                                         __half* __restrict__ vdst) {
+template <int D, int DT, bool ROLL>
+__global__ __launch_bounds__(256) void kv_prefill_copy_kernel(LayerView L, int n_slots, __half* __restrict__ kdst,
+                                                              __half* __restrict__ vdst) {
   constexpr int NB = D / kBlock;
   const size_t per_head = (size_t)n_slots * D / 16;  // 16-value chunks of K (and of V) per kv head
   const size_t total = per_head * L.kv_heads;
-  for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < 2 * total; c += (size_t)gridDim.x * blockDim.x) {
-    const bool isv = c >= total;
+  const size_t end = DT == KV_Q8 ? 2 * total : total;
+  for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < end; c += (size_t)gridDim.x * blockDim.x) {
+    const bool isv = DT == KV_Q8 && c >= total;
     const size_t cc = isv ? c - total : c;
     const int kvh = (int)(cc / per_head);
     const size_t e0 = (cc % per_head) * 16;  // element offset inside the kv head's region
     const size_t base = (size_t)kvh * L.cap * D;
-    const uint4 w = *(const uint4*)((const int8_t*)(isv ? L.v : L.k) + base + e0);
-    const uint32_t ww[4] = {w.x ^ 0x80808080u, w.y ^ 0x80808080u, w.z ^ 0x80808080u, w.w ^ 0x80808080u};
     _Float16 o[16];
     if (!isv) {
-      const int slot = (int)(e0 / D), d0 = (int)(e0 % D);
-      const float s = L.ks[((size_t)kvh * L.cap + slot) * NB + d0 / kBlock] * (1.0f / 127.0f);
+      // 16 dims of one key: consecutive ones, or 8 and their rotation partners
+      const int slot = (int)(e0 / D);
+      const int d0 = ROLL ? (int)(e0 % D) / 2 : (int)(e0 % D), d1 = ROLL ? d0 + D / 2 : d0 + 8;
+      float a[8], b[8];
+      if constexpr (DT == KV_Q8) {
+        const int8_t* row = (const int8_t*)L.k + base + (size_t)slot * D;
+        const uint2 wa = *(const uint2*)(row + d0), wb = *(const uint2*)(row + d1);
+        const float* ks = L.ks + ((size_t)kvh * L.cap + slot) * NB;
+        const float sa = ks[d0 / kBlock] * (1.0f / 127.0f), sb = ks[d1 / kBlock] * (1.0f / 127.0f);
+        const uint32_t ua[2] = {wa.x ^ 0x80808080u, wa.y ^ 0x80808080u}, ub[2] = {wb.x ^ 0x80808080u, wb.y ^ 0x80808080u};
 #pragma unroll
-      for (int i = 0; i < 16; i++) o[i] = q8_stage_f16((ww[i >> 2] >> (8 * (i & 3))) & 0xffu, s);
-      uint4* dst = (uint4*)(kdst + base + e0);
-      dst[0] = *(const uint4*)&o[0];
-      dst[1] = *(const uint4*)&o[8];
+        for (int i = 0; i < 8; i++) {
+          a[i] = q8_stage_f32((ua[i >> 2] >> (8 * (i & 3))) & 0xffu, sa);
+          b[i] = q8_stage_f32((ub[i >> 2] >> (8 * (i & 3))) & 0xffu, sb);
+        }
+      } else {
+        const _Float16* row = (const _Float16*)L.k + base + (size_t)slot * D;
+        const uint4 ha = *(const uint4*)(row + d0), hb = *(const uint4*)(row + d1);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          a[i] = (float)((const _Float16*)&ha)[i];
+          b[i] = (float)((const _Float16*)&hb)[i];
+        }
+      }
+      if constexpr (ROLL) {
+        const int Lg = slot < L.max_seq ? L.ring.logical(slot) : 0;
+        long ri = (L.rope_abs && Lg >= L.ring.sinks) ? (long)Lg + L.evicted : (long)Lg;
+        ri = ri < L.rope_positions ? ri : 0;  // a masked slot
+        const float* ct = L.cos_tab + (size_t)ri * (D / 2) + d0;
+        const float* st = L.sin_tab + (size_t)ri * (D / 2) + d0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const float x = a[i], y = b[i], cv = ct[i], sv = st[i];
+          a[i] = add_rn(mul_rn(x, cv), mul_rn(-y, sv));
+          b[i] = add_rn(mul_rn(y, cv), mul_rn(x, sv));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        o[i] = (_Float16)a[i];
+        o[8 + i] = (_Float16)b[i];
+      }
+      __half* dst = kdst + base + (size_t)slot * D;
+      *(uint4*)(dst + d0) = *(const uint4*)&o[0];
+      *(uint4*)(dst + d1) = *(const uint4*)&o[8];
     } else {
+      const uint4 w = *(const uint4*)((const int8_t*)L.v + base + e0);
+      const uint32_t ww[4] = {w.x ^ 0x80808080u, w.y ^ 0x80808080u, w.z ^ 0x80808080u, w.w ^ 0x80808080u};
       // 16 bytes of a V tile = 2 dims x the 8 slots of one panel
       const int t = (int)(e0 / ((size_t)kTile * D));
       const int wi = (int)(e0 % ((size_t)kTile * D));
@@ -146,13 +188,20 @@ __global__ __launch_bounds__(256) void kv_dequant_kernel(LayerView L, int n_slot
   }
 }
 
-hipError_t launch_kv_dequant_f16(const LayerView& L, int n_slots, void* kdst, void* vdst, hipStream_t st) {
-  if (L.dtype != KV_Q8 || n_slots <= 0 || n_slots % kTile || n_slots > L.cap) return hipErrorInvalidValue;
-  const size_t chunks = 2 * (size_t)n_slots * L.D / 16 * L.kv_heads;
-  const int grid = (int)((chunks + 255) / 256 < 4096 ? (chunks + 255) / 256 : 4096);
-  switch (L.D) {
-    case 128: hipLaunchKernelGGL((kv_dequant_kernel<128>), dim3(grid), dim3(256), 0, st, L, n_slots, (__half*)kdst, (__half*)vdst); break;
-    default: hipLaunchKernelGGL((kv_dequant_kernel<256>), dim3(grid), dim3(256), 0, st, L, n_slots, (__half*)kdst, (__half*)vdst); break;
+hipError_t launch_kv_prefill_copy(const LayerView& L, int n_slots, void* kdst, void* vdst, hipStream_t st) {
+  const bool q8 = L.dtype == KV_Q8, roll = L.ring.roll != 0;
+  if (n_slots <= 0 || n_slots % kTile || n_slots > L.cap || (!q8 && !(L.dtype == KV_F16 && roll))) return hipErrorInvalidValue;
+  const size_t chunks = (q8 ? 2 : 1) * (size_t)n_slots * L.D / 16 * L.kv_heads;
+  const dim3 grid((unsigned)((chunks + 255) / 256 < 4096 ? (chunks + 255) / 256 : 4096)), block(256);
+  __half *k = (__half*)kdst, *v = (__half*)vdst;
+  if (L.D == 128) {
+    if (!q8) hipLaunchKernelGGL((kv_prefill_copy_kernel<128, KV_F16, true>), grid, block, 0, st, L, n_slots, k, v);
+    else if (roll) hipLaunchKernelGGL((kv_prefill_copy_kernel<128, KV_Q8, true>), grid, block, 0, st, L, n_slots, k, v);
+    else hipLaunchKernelGGL((kv_prefill_copy_kernel<128, KV_Q8, false>), grid, block, 0, st, L, n_slots, k, v);
+  } else {
+    if (!q8) hipLaunchKernelGGL((kv_prefill_copy_kernel<256, KV_F16, true>), grid, block, 0, st, L, n_slots, k, v);
+    else if (roll) hipLaunchKernelGGL((kv_prefill_copy_kernel<256, KV_Q8, true>), grid, block, 0, st, L, n_slots, k, v);
+    else hipLaunchKernelGGL((kv_prefill_copy_kernel<256, KV_Q8, false>), grid, block, 0, st, L, n_slots, k, v);
   }
   return hipGetLastError();
 }

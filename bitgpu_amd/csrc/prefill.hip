@@ -20,8 +20,9 @@
 //             double-buffered with one barrier per step. An f16 cache is copied by the gfx950
 //             direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds: no registers, no VALU); q8
 //             codes are dequantized (code * block scale / 127) and sink-mode keys rotated at
-//             their slot position through registers, once per workgroup. Either way the next
-//             step's loads are in flight while this step computes.
+//             their slot position through registers, once per workgroup, where the launch does
+//             not run on an f16 copy that holds them so (prefill_wants_f16_copy). Either way the
+//             next step's loads are in flight while this step computes.
 //   pipeline  D=256 with f16 tiles (one wave per SIMD): K is staged one step ahead of V and
 //             iteration s runs the QK MFMAs of step s+1 with the exp2 / f16 / row-sum work of step
 //             s between them, then the PV MFMAs of step s -- the VALU work hides under MFMAs
@@ -76,6 +77,7 @@ struct PrefillParams {
   int n_qblocks;
   int n_scan_fixed;  // >0: scan this many physical slots for every block (sink mode after a wrap)
   int phys_limit;
+  int skip_t0, skip_n;  // steps skip_t0 .. + skip_n - 1 hold only slots that every row masks (sink mode)
   int mirror;        // pair items heavy / light over the one wave of the grid (see the kernel)
   // split-K: n_parts > 1 splits every item's key range into parts of part_steps steps, each
   // scanned by its own workgroup, which leaves its partial in pws for prefill_merge_kernel
@@ -113,7 +115,7 @@ struct StageRegs {
   float vsc[Q8 ? 8 : 1];      // q8: block scale of each of the 8 slots
 };
 
-template <int D, int DT, bool ROLL>
+template <int D, int DT, int ROLL>
 struct Stager {
   using C = PfCfg<D>;
   static constexpr int PH = D / 32;   // threads per key (16 dims per half each)
@@ -245,7 +247,7 @@ struct Stager {
         for (int e = 0; e < 8; e++) b[8 * i + e] = (float)h.e[e];
       }
     }
-    if constexpr (ROLL) {
+    if constexpr (ROLL == 1) {
       // pairs (i, i + D/2) at the key's rope position, f32 with one rounding per step (the
       // table rows are loaded here, not with the step's data, to keep registers for the MFMAs)
       const LayerView& L = p.L;
@@ -270,7 +272,7 @@ struct Stager {
       }
     }
     const int ca = cb / 8, cbb = (cb + D / 2) / 8;  // first chunk of each half
-    if constexpr (DT == KV_Q8 || ROLL) {
+    if constexpr (DT == KV_Q8 || ROLL == 1) {
       PH8 o;
 #pragma unroll
       for (int i = 0; i < 2; i++) {
@@ -309,11 +311,13 @@ struct Stager {
   }
 };
 
-template <int D, int DT, bool ROLL>
+// ROLL: 0 keys as stored, 1 sink-mode keys rotated at staging, 2 sink-mode keys already rotated (the
+// f16 copy); 1 and 2 mask by logical slot.
+template <int D, int DT, int ROLL>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillParams p) {
   using C = PfCfg<D>;
   constexpr int KT = C::KT, NSUB = C::NSUB, NC = C::NC, ND = C::ND, TILE = C::TILE;
-  constexpr bool DMA = DT == KV_F16 && !ROLL;
+  constexpr bool DMA = DT == KV_F16 && ROLL != 1;
   // software-pipelined steps where a wave has its SIMD to itself (D=256: 512 registers a wave);
   // D=128 runs two workgroups per CU, whose waves overlap one's softmax with the other's MFMAs
   constexpr bool PIPE = DMA && D == 256;
@@ -362,7 +366,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
   // key range of the block in KT-key steps
   const int last_q = min(s0 + p.QB, p.S) - 1;
   const int n_scan = p.n_scan_fixed > 0 ? p.n_scan_fixed : p.pos_base + last_q + 1;
-  const int steps_item = (n_scan + KT - 1) / KT;
+  const int steps_item = (n_scan + KT - 1) / KT - p.skip_n;
+  // first slot of step t: the steps over masked ring room are left out
+  auto slot0 = [&](int t) { return KT * (ROLL ? t + (t < p.skip_t0 ? 0 : p.skip_n) : t); };
   // this workgroup's steps [t0, steps) of the block's key range
   const int t0 = part * p.part_steps;
   const int steps = split ? min(t0 + p.part_steps, steps_item) : steps_item;
@@ -370,6 +376,29 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
   const int t_last = steps - 1;
   // the earliest key index any row of the block masks (causal diagonal or scan end)
   const int mask_from = min(min(p.pos_base + s0 + 1, n_scan), p.phys_limit);
+  // whether a row of the block masks a key of the step from slot j0. In a ring whose origin has
+  // moved the newest logical slot sits just before the oldest; elsewhere slots ascend.
+  auto step_masked = [&](int j0) {
+    if (!ROLL || ring.head == 0) return j0 + KT > mask_from;
+    const int last = j0 + KT - 1, newest = ring.sinks + ring.head - 1;
+    const int top = j0 <= newest && newest <= last ? ring.sinks + ring.W - 1 : ring.logical(last);
+    return last >= n_scan || last >= p.phys_limit || top > p.pos_base + s0;
+  };
+  // This lane's last unmasked slot of the step from j0, where one such slot is all there is to it:
+  // slots before the scan's end whose logical index (in a ring with a moved origin the slot less
+  // the origin, plus its size below the seam) is at most the row's position. False for a step
+  // that holds sinks or the seam.
+  auto last_slot = [&](int j0, int* thr) {
+    const int seam = ring.sinks + ring.head;
+    int lm = limit;
+    if (ROLL && ring.head != 0) {
+      if (j0 >= seam) lm = limit + ring.head;
+      else if (j0 >= ring.sinks && j0 + KT <= seam) lm = limit + ring.head - ring.W;
+      else return false;
+    }
+    *thr = min(lm, min(n_scan, p.phys_limit) - 1);
+    return true;
+  };
 
   // ---------------- prologue: Q and the first tile, loads issued together ----------------
   // each lane gathers its own Q^T operand (16 dims of one row per dim chunk)
@@ -382,12 +411,12 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
       qraw[2 * c + 1] = *(const float4*)(qr + 16 * c + 8 * g2 + 4);
     }
   }
-  const int j00 = t0 * KT;
+  const int j00 = slot0(t0);
   StageRegs<D, DT> R0;
   if constexpr (PIPE) {
     // K and V of the first step and K of the second (K is staged one step ahead of V)
     stg.dma(p, kvh, j00, k0, v0);
-    stg.dma_k(p, kvh, min(t0 + 1, t_last) * KT, k1);
+    stg.dma_k(p, kvh, slot0(min(t0 + 1, t_last)), k1);
   } else if constexpr (DMA) {
     stg.dma(p, kvh, j00, k0, v0);
   } else {
@@ -474,9 +503,21 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
     // mask S of step s1 into x and return its row max
     auto mask_max = [&](int s1, const floatx16 (&sacc)[NA]) {
       const bool live = s1 < steps;  // the look-ahead past the last step is all masked
-      const int j0 = (live ? s1 : 0) * KT;
+      const int j0 = live ? slot0(s1) : 0;
       float mt = -INFINITY;
-      if (!live || j0 + KT > mask_from) {
+      int thr = -(1 << 30);
+      const bool masked = !live || step_masked(j0);
+      if (masked && (!live || last_slot(j0, &thr))) {
+        thr -= j0 + 4 * g2;
+#pragma unroll
+        for (int u = 0; u < NSUB; u++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) {
+            const float v = 32 * u + 8 * (e >> 2) + (e & 3) <= thr ? sacc[u][e] : -INFINITY;
+            x[u][e] = v;
+            mt = fmaxf(mt, v);
+          }
+      } else if (ROLL && masked) {
 #pragma unroll
         for (int u = 0; u < NSUB; u++)
 #pragma unroll
@@ -484,7 +525,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
 #pragma unroll
             for (int e = 0; e < 4; e++) {
               const int P = j0 + 32 * u + 8 * k + 4 * g2 + e;
-              const bool ok = live && P < n_scan && P < p.phys_limit && P <= limit;
+              const bool ok = P < n_scan && P < p.phys_limit && ring.logical(P) <= limit;
               const float v = ok ? sacc[u][4 * k + e] : -INFINITY;
               x[u][4 * k + e] = v;
               mt = fmaxf(mt, v);
@@ -522,8 +563,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
     __syncthreads();  // the first K buffer and the Q operand area are free
 
     auto pstep = [&](int s, const _Float16* kn, const _Float16* vc, _Float16* kd, _Float16* vd) {
-      stg.dma_k(p, kvh, min(s + 2, t_last) * KT, kd);
-      stg.dma_v(p, kvh, min(s + 1, t_last) * KT, vd);
+      stg.dma_k(p, kvh, slot0(min(s + 2, t_last)), kd);
+      stg.dma_v(p, kvh, slot0(min(s + 1, t_last)), vd);
       floatx16 sacc[NA];
       PH8 pb[NSUB][2];
       qk(std::true_type{}, kn, sacc, pb);
@@ -562,7 +603,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
   } else {
     // ---------------- one step: stage step s+1 into (kn, vn), compute step s from (kc, vc) ----------------
     auto step = [&](int s, const _Float16* kc, const _Float16* vc, _Float16* kn, _Float16* vn) {
-      const int jn = min(s + 1, t_last) * KT;
+      const int jn = slot0(min(s + 1, t_last));
       StageRegs<D, DT> R;
       if constexpr (DMA) {
         stg.dma(p, kvh, jn, kn, vn);
@@ -573,7 +614,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
         __builtin_amdgcn_sched_barrier(0);
       }
 
-      const int j0 = s * KT;
+      const int j0 = slot0(s);
       // S^T = K Q^T
       // one 32-key sub-tile (D=256): two accumulators over even / odd dim chunks, so the QK
       // MFMAs form two independent chains
@@ -613,7 +654,19 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
       // mask + online softmax (row = this lane's n)
       float x[NSUB][16];
       float mt = -INFINITY;
-      if (ROLL || j0 + KT > mask_from) {
+      // (the plain cache's kernel keeps the comparison a key: the other schedules 6 % slower there)
+      int thr;
+      if (ROLL && step_masked(j0) && last_slot(j0, &thr)) {
+        thr -= j0 + 4 * g2;
+#pragma unroll
+        for (int u = 0; u < NSUB; u++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) {
+            const float v = 32 * u + 8 * (e >> 2) + (e & 3) <= thr ? sacc[u][e] : -INFINITY;
+            x[u][e] = v;
+            mt = fmaxf(mt, v);
+          }
+      } else if (step_masked(j0)) {
 #pragma unroll
         for (int u = 0; u < NSUB; u++)
 #pragma unroll
@@ -815,7 +868,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
   const bool row_ok = r < p.QB * p.G && qi < p.S;
   const int last_q = min(s0 + p.QB, p.S) - 1;
   const int n_scan = p.n_scan_fixed > 0 ? p.n_scan_fixed : p.pos_base + last_q + 1;
-  const int steps_item = (n_scan + KT - 1) / KT;
+  const int steps_item = (n_scan + KT - 1) / KT - p.skip_n;
   const int np = (steps_item + p.part_steps - 1) / p.part_steps;  // parts that scanned keys
   const size_t pstride = (size_t)p.split_waves;                   // per part, in (wave) units
   const size_t pi0 = (size_t)item * p.n_parts * p.split_waves + wave;
@@ -899,6 +952,59 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
   }
 }
 
+// The merge of up to kMergeParts parts: workgroup (item, wave, 32-dim chunk), a wave a slot of the
+// chunk, a lane its column of every part, all loaded before any is used: no barrier, and the four
+// waves' 32-byte pieces of a row fill its 128-byte line. (The kernel above, a workgroup a slot,
+// took 20 us for 128 items of two parts, 25 MB; this one 8, the other's markers aside.)
+constexpr int kMergeParts = 8;
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_few_kernel(PrefillParams p) {
+  constexpr int KT = PfCfg<D>::KT, ND = D / 32, NSL = 4 * ND;
+  const int KV = p.L.kv_heads;
+  const int dc = blockIdx.x % ND, iw = blockIdx.x / ND;
+  const int item = iw / p.split_waves, wave = iw % p.split_waves;
+  const int lane = threadIdx.x & 63, sl = 4 * dc + (threadIdx.x >> 6);
+  const int kvh = item % KV;
+  const int qb = p.n_qblocks - 1 - item / KV;
+  const int s0 = qb * p.QB;
+  const int n = lane & 31, g2 = lane >> 5, r = wave * 32 + n;
+  const int qi = s0 + r / p.G, h = kvh * p.G + r % p.G;
+  if (r >= p.QB * p.G || qi >= p.S) return;
+  const int last_q = min(s0 + p.QB, p.S) - 1;
+  const int n_scan = p.n_scan_fixed > 0 ? p.n_scan_fixed : p.pos_base + last_q + 1;
+  const int np = ((n_scan + KT - 1) / KT - p.skip_n + p.part_steps - 1) / p.part_steps;  // parts that scanned keys
+  const size_t pi0 = (size_t)item * p.n_parts * p.split_waves + wave;
+  float2 ml[kMergeParts];
+  float4 v[kMergeParts];
+  float M = -INFINITY;
+#pragma unroll
+  for (int q = 0; q < kMergeParts; q++) {
+    const size_t pi = pi0 + (size_t)min(q, np - 1) * p.split_waves;
+    ml[q] = p.pml[pi * 64 + lane];
+    v[q] = p.pws[(pi * NSL + sl) * 64 + lane];
+  }
+  float4 gv = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int d = 32 * dc + 8 * (sl & 3) + 4 * g2;
+  if (p.gate) gv = *(const float4*)(p.gate + ((size_t)qi * p.H + h) * p.gate_stride + d);
+#pragma unroll
+  for (int q = 0; q < kMergeParts; q++) M = fmaxf(M, ml[q].x);
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  float lt = 0.0f;
+#pragma unroll
+  for (int q = 0; q < kMergeParts; q++) {
+    const float w = q < np ? __builtin_amdgcn_exp2f(ml[q].x - M) : 0.0f;
+    o.x += v[q].x * w;
+    o.y += v[q].y * w;
+    o.z += v[q].z * w;
+    o.w += v[q].w * w;
+    lt += ml[q].y * w;
+  }
+  o = make_float4(o.x / lt, o.y / lt, o.z / lt, o.w / lt);
+  if (p.gate)
+    o = make_float4(o.x / (1.0f + expf(-gv.x)), o.y / (1.0f + expf(-gv.y)), o.z / (1.0f + expf(-gv.z)), o.w / (1.0f + expf(-gv.w)));
+  *(float4*)(p.out + ((size_t)qi * p.H + h) * D + d) = o;
+}
+
 bool prefill_supported(const LayerView& L, int S, int H) {
   if (L.dtype == KV_F32) return false;
   if (L.D != 128 && L.D != 256) return false;
@@ -908,11 +1014,31 @@ bool prefill_supported(const LayerView& L, int S, int H) {
 
 bool prefill_wants_f16_copy(const LayerView& L, int S, int H) {
   // each K/V tile is staged once per query block (128 rows of (query, head) pairs); from four
-  // blocks on, one dequantizing pass plus the f16 direct-to-LDS staging costs less
-  if (L.dtype != KV_Q8 || L.ring.roll) return false;
+  // blocks on, one dequantizing pass plus the f16 direct-to-LDS staging costs less. Sink-mode
+  // keys cost more to stage (a step that rotates takes 3 us against 1), so from two blocks: 500
+  // rows over 3,500 slots 139 us -> 62, 100 rows 47 -> 29, 40 rows (two blocks) 31 -> 26.
+  if (L.dtype == KV_F32 || (L.dtype == KV_F16 && !L.ring.roll)) return false;
   const int G = H / L.kv_heads;
   const int QB = 128 / G;
-  return (S + QB - 1) / QB >= 4;
+  return (S + QB - 1) / QB >= (L.ring.roll ? 2 : 4);
+}
+
+// Sink mode after the ring origin has moved: the steps that hold only slots past every row's
+// position (the room eviction left) are not scanned, the longest run of whole ones.
+static void pf_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n) {
+  *t0 = *n = 0;
+  const int first = pos_base + S, sk = L.ring.sinks, W = L.ring.W;  // first logical slot no row sees
+  if (!L.ring.roll || L.ring.head == 0 || first < sk || first >= sk + W) return;
+  auto take = [&](int x, int y) {  // physical slots [x, y)
+    const int a = (x + KT - 1) / KT, b = y / KT;
+    if (b - a > *n) {
+      *t0 = a;
+      *n = b - a;
+    }
+  };
+  const int a = sk + (first - sk + L.ring.head) % W, len = sk + W - first;
+  take(a, std::min(a + len, sk + W));
+  if (a + len > sk + W) take(sk, a + len - W);
 }
 
 // D=128 runs two workgroups a CU (64 KB of LDS and 256 registers a wave each). A D=128 grid that
@@ -927,7 +1053,7 @@ static bool pf_mirror(const LayerView& L, int n_items, int num_cus) { return L.D
 // least kPfMinPartSteps steps, at most one round of workgroups. The part count is the cheapest by
 // a cost model in microseconds, its constants measured: a step takes about 1 us of a CU, 2.1 us
 // where a D=128 CU runs two workgroups; a part's partial (32 KB a wave at D=256, 16 KB at D=128)
-// is written and read at about 4.5 TB/s, and the merge kernel adds about 6 us. So a short prompt stays whole
+// is written and read at about 4.5 TB/s, and the merge kernel adds about 5 us. So a short prompt stays whole
 // (S=500: 14.8 us, 31 split in two) and a turn of 333 tokens after 12,000 takes five parts (184 ->
 // 107 us; two 127, three 135), 300 after 3,000 at D=256 four (129 -> 68 us; two 86, eight 83).
 // Both entry points use the same plan (the allocation-free one's scratch holds every plan's
@@ -944,7 +1070,9 @@ static PfSplitPlan pf_split_plan(const LayerView& L, int S, int H, int pos_base,
   const int KT = L.D == 128 ? PfCfg<128>::KT : PfCfg<256>::KT;
   const int per_cu = L.D == 128 ? 2 : 1;  // workgroups a CU holds
   const long slots = (L.ring.roll && L.ring.head != 0) ? (long)L.max_seq : (long)pos_base + S;
-  const int steps_max = (int)((slots + KT - 1) / KT);
+  int skip_t0, skip_n;
+  pf_skip(L, S, pos_base, KT, &skip_t0, &skip_n);
+  const int steps_max = (int)((slots + KT - 1) / KT) - skip_n;
   // partials only for the waves holding rows: (query, head) rows of a block, 32 a wave
   const int waves = std::min(4, (std::min(QB, S) * G + 31) / 32);
   const size_t part_bytes = (size_t)waves * 4 * (L.D / 32) * 64 * sizeof(float4);
@@ -958,7 +1086,7 @@ static PfSplitPlan pf_split_plan(const LayerView& L, int S, int H, int pos_base,
   for (int np = 2; np <= P; np++) {
     const int ps = (steps_max + np - 1) / np;
     if ((steps_max + ps - 1) / ps != np) continue;  // the same split as fewer parts
-    const float t = ps * (n_items * np > num_cus ? 2.1f : 1.0f) + n_items * np * us_part + 6.0f;
+    const float t = ps * (n_items * np > num_cus ? 2.1f : 1.0f) + n_items * np * us_part + 5.0f;
     if (t < best) {
       best = t;
       r.n_parts = np;
@@ -982,11 +1110,13 @@ bool prefill_can_split(const LayerView& L, int S, int H, int num_cus) {
   return 2 * n_items <= (L.D == 128 ? 2 : 1) * num_cus;
 }
 
-template <int D, int DT, bool ROLL>
+template <int D, int DT, int ROLL>
 static hipError_t launch_pf(const PrefillParams& p, hipStream_t st) {
   const int n_items = p.n_qblocks * p.L.kv_heads;
   hipLaunchKernelGGL((prefill_kernel<D, DT, ROLL>), dim3(n_items * p.n_parts), dim3(256), 0, st, p);
-  if (p.n_parts > 1)
+  if (p.n_parts > 1 && p.n_parts <= kMergeParts)
+    hipLaunchKernelGGL((prefill_merge_few_kernel<D>), dim3(n_items * p.split_waves * (D / 32)), dim3(256), 0, st, p);
+  else if (p.n_parts > 1)
     hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3(n_items * p.split_waves * 4 * (D / 32)), dim3(256), 0, st, p);
   return hipGetLastError();
 }
@@ -1007,6 +1137,7 @@ hipError_t launch_attention_prefill(const LayerView& L, const AttnArgs& a, hipSt
   p.n_qblocks = (a.S + p.QB - 1) / p.QB;
   p.n_scan_fixed = (L.ring.roll && L.ring.head != 0) ? L.max_seq : 0;
   p.phys_limit = L.ring.roll ? L.max_seq : L.cap;
+  pf_skip(L, a.S, a.pos_base, L.D == 128 ? PfCfg<128>::KT : PfCfg<256>::KT, &p.skip_t0, &p.skip_n);
   p.mirror = pf_mirror(L, p.n_qblocks * L.kv_heads, a.num_cus);
   p.n_parts = 1;
   p.part_steps = 0;
@@ -1023,13 +1154,16 @@ hipError_t launch_attention_prefill(const LayerView& L, const AttnArgs& a, hipSt
     p.pml = (float2*)a.pf_ml;
     p.mirror = 0;
   }
-  const bool roll = L.ring.roll != 0;
+  const int roll = !L.ring.roll ? 0 : a.k_rotated ? 2 : 1;
+  if (roll == 2 && L.dtype != KV_F16) return hipErrorInvalidValue;
   if (L.D == 128) {
-    if (L.dtype == KV_Q8) return roll ? launch_pf<128, KV_Q8, true>(p, st) : launch_pf<128, KV_Q8, false>(p, st);
-    return roll ? launch_pf<128, KV_F16, true>(p, st) : launch_pf<128, KV_F16, false>(p, st);
+    if (L.dtype == KV_Q8) return roll ? launch_pf<128, KV_Q8, 1>(p, st) : launch_pf<128, KV_Q8, 0>(p, st);
+    return roll == 2 ? launch_pf<128, KV_F16, 2>(p, st)
+                     : roll ? launch_pf<128, KV_F16, 1>(p, st) : launch_pf<128, KV_F16, 0>(p, st);
   }
-  if (L.dtype == KV_Q8) return roll ? launch_pf<256, KV_Q8, true>(p, st) : launch_pf<256, KV_Q8, false>(p, st);
-  return roll ? launch_pf<256, KV_F16, true>(p, st) : launch_pf<256, KV_F16, false>(p, st);
+  if (L.dtype == KV_Q8) return roll ? launch_pf<256, KV_Q8, 1>(p, st) : launch_pf<256, KV_Q8, 0>(p, st);
+  return roll == 2 ? launch_pf<256, KV_F16, 2>(p, st)
+                   : roll ? launch_pf<256, KV_F16, 1>(p, st) : launch_pf<256, KV_F16, 0>(p, st);
 }
 
 }  // namespace bg

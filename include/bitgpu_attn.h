@@ -19,7 +19,7 @@
  *   - Kernels never allocate. Host-side allocations happen only in bg_kv_create, bg_kv_grow,
  *     bg_attention_reserve, lazily on the first bg_attention that needs more workspace (split
  *     partials, at most 33 MiB of them for a split-K prefill, which runs unsplit where they cannot
- *     be had) or, for a q8 cache, the f16 copy a long prefill runs on, and in the snapshot
+ *     be had) or, for a q8 or sink-mode cache, the f16 copy a long prefill runs on, and in the snapshot
  *     transfers (a staging buffer kept by the cache, grown when a larger region is transferred).
  *   - The decode kernel's split merge waits a bounded time for the partials of its own grid.
  *     If a wait gives up (the GPU shared with work that keeps the grid from running at once),
@@ -251,8 +251,9 @@ int32_t bg_attention(bg_kv_cache* cache, int32_t layer, const float* q, int32_t 
  * capture, tight serving loops, harnesses that forbid allocation. Same arguments and results as
  * bg_attention, but it allocates nothing: the split partials of the decode kernel (8 MiB per GPU)
  * and of a split-K prefill (33 MiB, as much as any plan needs) live in a file-scope device array,
- * held until the process ends, instead of the cache's workspace; a q8 prefill stages its tiles
- * in-kernel instead of through the f16 copy (the same values: identical output); an f32 cache runs the exact-f32 kernel of one wave per
+ * held until the process ends, instead of the cache's workspace; a q8 or sink-mode prefill
+ * dequantizes and rotates in-kernel instead of through the f16 copy (the same values: identical
+ * output); an f32 cache runs the exact-f32 kernel of one wave per
  * (query, head), which keeps no partials (agrees with bg_attention to f32 rounding). A decode
  * launch whose partials would exceed its 8 MiB is rejected with BG_E_INVALID before anything runs.
  * The first call on a device sets the array up (a fill kernel, synchronized) and must not be
@@ -264,8 +265,8 @@ int32_t bg_attention_noalloc(bg_kv_cache* cache, int32_t layer, const float* q, 
                              float* out, void* stream);
 
 /* Pre-size the split-K workspace for up to S query rows of H heads (otherwise sized on first
- * use), and for a q8 cache whose prefill of S rows runs on an f16 copy of the attended slots,
- * allocate that copy; for a prefill of S rows that can split along the key range, its partials
+ * use), and for a q8 or sink-mode cache whose prefill of S rows runs on an f16 copy of the
+ * attended slots, allocate that copy; for a prefill of S rows that can split along the key range, its partials
  * and (m, l) buffer. Call before capturing bg_attention into a HIP graph (a launch under capture
  * cannot allocate). A later call that needs a larger workspace allocates a new one and keeps the
  * old one until bg_kv_destroy, so launches captured before stay valid. */
