@@ -739,6 +739,11 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
 
 int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
   if (!c || S < 1 || H < 1 || H % c->kv_heads) return fail(BG_E_INVALID, "bg_attention_reserve: bad arguments");
+  if (c->dtype == BG_KV_F32 && !bg::f32_split_supported(view(c, 0), S, H)) {
+    if (!ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
+      return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
+    return BG_OK;
+  }
   if (c->dtype != BG_KV_F32 && !bg::decode_preferred(view(c, 0), S, H)) {
     if (bg::prefill_wants_f16_copy(view(c, 0), S, H)) {
       int32_t rc = ensure_prefill_copy(c);
@@ -820,6 +825,12 @@ int32_t bg_attention(bg_kv_cache* c, int32_t layer, const float* q, int32_t S, i
     a.ws_floats = c->ws_floats;
     e = bg::launch_attention_f32_split(L, a, st);
   } else if (c->dtype == BG_KV_F32) {
+    const size_t pf = bg::f32_prefill_floats(L, S, H, pos_base, c->num_cus);
+    if (pf > 0 && ensure_prefill_split(c, pf, st)) {
+      a.pf_o = c->pf_o;
+      a.pf_ml = c->pf_ml;
+      a.pf_floats = c->pf_floats;
+    }
     e = bg::launch_attention_f32(L, a, st);
   } else if (bg::decode_preferred(L, S, H)) {
     int32_t rc = ensure_workspace(c, S, H);
@@ -905,8 +916,12 @@ int32_t bg_attention_noalloc(bg_kv_cache* c, int32_t layer, const float* q, int3
   if (rc != BG_OK) return rc;
   LayerView L = view(c, layer);
   bg::AttnArgs a = attention_args(c, q, S, H, pos_base, scale, gate, gate_stride, out);
+  // a prefill that splits its key ranges keeps its partials in the scratch, which holds every plan's
+  a.pf_o = (float*)((char*)ptr + kScratchBytes);
+  a.pf_floats = bg::kPfSplitBytes / sizeof(float);
+  a.pf_ml = (float*)((char*)ptr + kScratchBytes + bg::kPfSplitBytes);
   if (c->dtype == BG_KV_F32) {
-    // the f32 kernels run without partials here (the matrix-core kernel for every shape)
+    // the matrix-core kernel for every shape
     e = bg::launch_attention_f32(L, a, st);
   } else if (bg::decode_preferred(L, S, H)) {
     bg::DecodePlan pl;
@@ -920,11 +935,7 @@ int32_t bg_attention_noalloc(bg_kv_cache* c, int32_t layer, const float* q, int3
     a.ws_floats = kScratchBytes / sizeof(float);
     e = bg::launch_attention_decode(L, a, st);
   } else if (bg::prefill_supported(L, S, H)) {
-    // a q8 cache is staged in-kernel (no f16 copy): the same values, so the same results; a
-    // split-K prefill keeps its partials in the scratch, which holds every plan's
-    a.pf_o = (float*)((char*)ptr + kScratchBytes);
-    a.pf_floats = bg::kPfSplitBytes / sizeof(float);
-    a.pf_ml = (float*)((char*)ptr + kScratchBytes + bg::kPfSplitBytes);
+    // a q8 or sink-mode cache is converted in-kernel (no f16 copy): the same values and results
     e = bg::launch_attention_prefill(L, a, st);
   } else {
     return fail(BG_E_UNSUPPORTED, "bg_attention_noalloc: no kernel for S %d, heads %d", S, H);

@@ -160,6 +160,14 @@ constexpr int kPfMaxParts = 512;
 // floats of the partials a prefill launch uses at pos_base (0: the launch does not split); whether
 // S rows of H heads can split at any pos_base (the partials are then at most kPfSplitBytes)
 size_t prefill_workspace_floats(const LayerView& L, int S, int H, int pos_base, int num_cus);
+// merges the partials of `waves` 32-row waves an item, parts of part_steps 64-key (head_dim 128) or
+// 32-key (256) steps
+hipError_t launch_prefill_merge(const LayerView& L, const AttnArgs& a, int QB, int n_parts, int part_steps, int waves,
+                                int n_scan_fixed, int skip_n, hipStream_t st);
+// the KT-slot steps *t0 .. + *n - 1 of a wrapped ring that hold only slots past S rows at pos_base
+void prefill_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n);
+// floats of the partials an f32 prefill uses at pos_base (0: none)
+size_t f32_prefill_floats(const LayerView& L, int S, int H, int pos_base, int num_cus);
 bool prefill_can_split(const LayerView& L, int S, int H, int num_cus);
 
 }  // namespace bg

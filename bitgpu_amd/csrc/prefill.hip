@@ -1025,7 +1025,7 @@ bool prefill_wants_f16_copy(const LayerView& L, int S, int H) {
 
 // Sink mode after the ring origin has moved: the steps that hold only slots past every row's
 // position (the room eviction left) are not scanned, the longest run of whole ones.
-static void pf_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n) {
+void prefill_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n) {
   *t0 = *n = 0;
   const int first = pos_base + S, sk = L.ring.sinks, W = L.ring.W;  // first logical slot no row sees
   if (!L.ring.roll || L.ring.head == 0 || first < sk || first >= sk + W) return;
@@ -1071,7 +1071,7 @@ static PfSplitPlan pf_split_plan(const LayerView& L, int S, int H, int pos_base,
   const int per_cu = L.D == 128 ? 2 : 1;  // workgroups a CU holds
   const long slots = (L.ring.roll && L.ring.head != 0) ? (long)L.max_seq : (long)pos_base + S;
   int skip_t0, skip_n;
-  pf_skip(L, S, pos_base, KT, &skip_t0, &skip_n);
+  prefill_skip(L, S, pos_base, KT, &skip_t0, &skip_n);
   const int steps_max = (int)((slots + KT - 1) / KT) - skip_n;
   // partials only for the waves holding rows: (query, head) rows of a block, 32 a wave
   const int waves = std::min(4, (std::min(QB, S) * G + 31) / 32);
@@ -1110,14 +1110,45 @@ bool prefill_can_split(const LayerView& L, int S, int H, int num_cus) {
   return 2 * n_items <= (L.D == 128 ? 2 : 1) * num_cus;
 }
 
+template <int D>
+static void launch_merge(const PrefillParams& p, hipStream_t st) {
+  const int waves = p.n_qblocks * p.L.kv_heads * p.split_waves;
+  if (p.n_parts <= kMergeParts)
+    hipLaunchKernelGGL((prefill_merge_few_kernel<D>), dim3(waves * (D / 32)), dim3(256), 0, st, p);
+  else
+    hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3(waves * 4 * (D / 32)), dim3(256), 0, st, p);
+}
+
+hipError_t launch_prefill_merge(const LayerView& L, const AttnArgs& a, int QB, int n_parts, int part_steps, int waves,
+                                int n_scan_fixed, int skip_n, hipStream_t st) {
+  PrefillParams p{};
+  p.L = L;
+  p.S = a.S;
+  p.H = a.H;
+  p.G = a.H / L.kv_heads;
+  p.QB = QB;
+  p.pos_base = a.pos_base;
+  p.gate = a.gate;
+  p.gate_stride = a.gate_stride;
+  p.out = a.out;
+  p.n_qblocks = (a.S + QB - 1) / QB;
+  p.n_scan_fixed = n_scan_fixed;
+  p.skip_n = skip_n;
+  p.n_parts = n_parts;
+  p.part_steps = part_steps;
+  p.split_waves = waves;
+  p.pws = (float4*)a.pf_o;
+  p.pml = (float2*)a.pf_ml;
+  if (L.D == 128) launch_merge<128>(p, st);
+  else launch_merge<256>(p, st);
+  return hipGetLastError();
+}
+
 template <int D, int DT, int ROLL>
 static hipError_t launch_pf(const PrefillParams& p, hipStream_t st) {
   const int n_items = p.n_qblocks * p.L.kv_heads;
   hipLaunchKernelGGL((prefill_kernel<D, DT, ROLL>), dim3(n_items * p.n_parts), dim3(256), 0, st, p);
-  if (p.n_parts > 1 && p.n_parts <= kMergeParts)
-    hipLaunchKernelGGL((prefill_merge_few_kernel<D>), dim3(n_items * p.split_waves * (D / 32)), dim3(256), 0, st, p);
-  else if (p.n_parts > 1)
-    hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3(n_items * p.split_waves * 4 * (D / 32)), dim3(256), 0, st, p);
+  if (p.n_parts > 1) launch_merge<D>(p, st);
   return hipGetLastError();
 }
 
@@ -1137,7 +1168,7 @@ hipError_t launch_attention_prefill(const LayerView& L, const AttnArgs& a, hipSt
   p.n_qblocks = (a.S + p.QB - 1) / p.QB;
   p.n_scan_fixed = (L.ring.roll && L.ring.head != 0) ? L.max_seq : 0;
   p.phys_limit = L.ring.roll ? L.max_seq : L.cap;
-  pf_skip(L, a.S, a.pos_base, L.D == 128 ? PfCfg<128>::KT : PfCfg<256>::KT, &p.skip_t0, &p.skip_n);
+  prefill_skip(L, a.S, a.pos_base, L.D == 128 ? PfCfg<128>::KT : PfCfg<256>::KT, &p.skip_t0, &p.skip_n);
   p.mirror = pf_mirror(L, p.n_qblocks * L.kv_heads, a.num_cus);
   p.n_parts = 1;
   p.part_steps = 0;

@@ -253,8 +253,8 @@ int32_t bg_attention(bg_kv_cache* cache, int32_t layer, const float* q, int32_t 
  * and of a split-K prefill (33 MiB, as much as any plan needs) live in a file-scope device array,
  * held until the process ends, instead of the cache's workspace; a q8 or sink-mode prefill
  * dequantizes and rotates in-kernel instead of through the f16 copy (the same values: identical
- * output); an f32 cache runs the exact-f32 kernel of one wave per
- * (query, head), which keeps no partials (agrees with bg_attention to f32 rounding). A decode
+ * output); an f32 cache runs the f32 matrix-core kernel for every shape, decode included
+ * (agrees with bg_attention to f32 rounding). A decode
  * launch whose partials would exceed its 8 MiB is rejected with BG_E_INVALID before anything runs.
  * The first call on a device sets the array up (a fill kernel, synchronized) and must not be
  * under graph capture (BG_E_STATE). Every call on one GPU shares that GPU's array: calls that

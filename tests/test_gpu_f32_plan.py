@@ -1,0 +1,52 @@
+"""GPU: f32 prefill at head_dim 128 over its plans -- waves sharing 32, 64 and 128 rows, key ranges
+split over workgroups, heads per kv head that do not divide 32, wrapped sink rings -- against the
+oracle (max-abs 1e-4, the bar for f32 storage)."""
+import numpy as np
+import pytest
+
+from oracle import ref
+from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc
+from tests.test_gpu_sink_copy import _ring
+from tests.test_gpu_split_prefill import _case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,KV,ctx,S,gate", [
+    (16, 8, 0, 9, False),       # 18 rows a kv head: one partial 32-row item
+    (16, 8, 0, 333, True),      # 32-row items, a ragged end
+    (24, 8, 0, 129, False),     # 3 heads a kv head: queries across row groups
+    (12, 1, 700, 40, False),    # 12 heads a kv head
+    (100, 1, 50, 3, True),      # 100 heads: a query an item
+    (32, 8, 5000, 9, False),    # a verify after a long context: parts over workgroups
+    (16, 2, 4001, 70, True),
+    (32, 8, 2000, 150, False),
+])
+def test_f32_plans(dev, H, KV, ctx, S, gate):
+    c, _, q, g = _case("f32", H, KV, 128, ctx + S, S, seed=H + ctx + S, gate=gate)
+    out = run_attention(c, 0, q, ctx, gate=g)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    want = ref.gated_attention(q, kk, vv, g, ctx) if gate else ref.attention(q, kk, vv, ctx)
+    assert np.abs(out - want).max() <= 1e-4
+    assert np.array_equal(run_attention_noalloc(c, 0, q, ctx, gate=g), out)
+    c.close()
+
+
+def test_f32_wide_rows(dev):
+    """128-row items, a wave its own rows (a long prompt), on a sample of the rows."""
+    H, KV, S = 32, 8, 2048
+    c, _, q, _ = _case("f32", H, KV, 128, S, S, seed=1, gate=False)
+    out = run_attention(c, 0, q, 0)
+    kk, vv = cached_values(c, 0, 0, S)
+    for r in (0, 31, 777, 2040):
+        want = ref.attention(q[r:r + 8], kk[:r + 8], vv[:r + 8], r)
+        assert np.abs(out[r:r + 8] - want).max() <= 1e-4
+    c.close()
+
+
+@pytest.mark.parametrize("window,moves,fill,S,mode", [
+    (1000, (300,), 700, 60, "slot"), (1000, (900,), 700, 100, "absolute"), (1020, (316,), 960, 64, "slot")])
+def test_f32_sink_ring(dev, window, moves, fill, S, mode):
+    c, q, want = _ring("f32", 32, 8, 128, window, moves, fill, S, mode)
+    assert np.abs(run_attention(c, 0, q, fill) - want).max() <= 1e-4
+    c.close()
