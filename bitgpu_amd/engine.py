@@ -26,6 +26,11 @@ import math
 
 import numpy as np
 
+try:
+    import torch
+except ImportError:  # the host-only functions (tables, plans, snapshot checks) need no torch
+    torch = None
+
 from ._lib import (BG_E_INVALID, BG_E_STATE, BG_K, BG_KSCALE, BG_ROPE_ABSOLUTE, BG_ROPE_SLOT, BG_V, BG_VSCALE,
                    KV_DTYPES, BitgpuError, check, lib)
 
@@ -34,9 +39,19 @@ __all__ = ["KvCache", "attention", "qkv_prologue", "layer_attention", "hybrid_fu
            "qkv_proj_prologue", "decode_attention_block"]
 
 
-def _stream():
-    import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# A decode step makes two to four of these calls a layer on kernels of 4 to 13 us, so what a call
+# costs on the host is the step's time: pointers and streams go to ctypes as plain integers and the
+# current stream is asked for as one, not through a Stream object (2.9 us). layer_attention 22.7 ->
+# 13.9 us a call (the two C calls alone 7).
+_getDevice = getattr(getattr(torch, "_C", None), "_cuda_getDevice", None)
+_getRawStream = getattr(getattr(torch, "_C", None), "_cuda_getCurrentRawStream", None)
+
+
+def _stream() -> int:
+    """The current device's current stream (hipStream_t as an integer)."""
+    if _getRawStream is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _getRawStream(_getDevice())
 
 
 def _ptr(t):
@@ -46,14 +61,28 @@ def _ptr(t):
         raise ValueError("bitgpu_amd: expected a device (cuda) tensor")
     if not t.is_contiguous():
         raise ValueError("bitgpu_amd: expected a contiguous tensor")
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _f32(t, name):
-    import torch
-    if t.dtype != torch.float32:
+    if t.dtype is not torch.float32:
         raise TypeError(f"bitgpu_amd: {name} must be float32, got {t.dtype}")
     return t
+
+
+def _rows_like(t, S, H, D):
+    """An uninitialized f32 [S, H, D] on t's device (t is f32 already)."""
+    return torch.empty_like(t) if t.shape == (S, H, D) and t.is_contiguous() else t.new_empty((S, H, D))
+
+
+_scales: dict = {}  # head_dim -> the dense kernels' softmax scale, f32 1 / sqrt(D) (attention_sg.wgsl:24)
+
+
+def _dense_scale(D):
+    s = _scales.get(D)
+    if s is None:
+        s = _scales[D] = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+    return s
 
 
 def rope_tables(theta: float, rot_dim: int, positions: int, yarn: dict | None = None):
@@ -324,21 +353,22 @@ def attention(cache: KvCache, li: int, qr, S: int, H: int, pos_base: int, scale:
               gate=None, gate_stride: int | None = None, out=None):
     """runN(ATT, [S,H,KV,D,posBase,Ltot], attIns(qr, li), att, S*H) (src/engine.ts:1543,1579-1580);
     with ``gate`` the hybrid's attention_online_cache + gate_sigmoid (1486-1491)."""
-    import torch
     D = cache.head_dim
     _f32(qr, "q")
     if qr.numel() != S * H * D:
         raise ValueError("bitgpu_amd: q must hold S*H*head_dim values")
     if out is None:
-        out = torch.empty((S, H, D), dtype=torch.float32, device=qr.device)
+        out = _rows_like(qr, S, H, D)
     if scale is None:
-        scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))  # attention_sg.wgsl:24
+        scale = _dense_scale(D)
     gs = 0
     if gate is not None:
         _f32(gate, "gate")
         gs = int(gate_stride if gate_stride is not None else D)
-    check(lib().bg_attention(cache.handle, li, _ptr(qr), S, H, int(pos_base), float(scale), _ptr(gate), gs,
-                             _ptr(out), _stream()))
+    rc = lib().bg_attention(cache._h, li, _ptr(qr), S, H, int(pos_base), float(scale), _ptr(gate), gs, _ptr(out),
+                            _stream())
+    if rc:
+        check(rc)
     return out
 
 
@@ -346,17 +376,18 @@ def qkv_prologue(cache: KvCache, li: int, q, k, v, S: int, H: int, q_gamma, k_ga
                  cos_tab, sin_tab, rot_dim: int, pos0: int, slot0: int, q_stride: int | None = None,
                  q_out=None):
     """Fused q/k RMSNorm + RoPE + K/V cache write (see include/bitgpu_attn.h bg_qkv_prologue)."""
-    import torch
     D = cache.head_dim
-    if q is not None and q_out is None:
-        q_out = torch.empty((S, H, D), dtype=torch.float32, device=q.device)
     for t, nm in ((q, "q"), (k, "k"), (v, "v"), (q_gamma, "q_gamma"), (k_gamma, "k_gamma")):
         if t is not None:
             _f32(t, nm)
-    check(lib().bg_qkv_prologue(cache.handle, li, _ptr(q), int(q_stride or D), _ptr(k), _ptr(v), S, H,
-                                _ptr(q_gamma), _ptr(k_gamma), float(eps), _ptr(cos_tab), _ptr(sin_tab),
-                                int(cos_tab.shape[0]) if cos_tab is not None else 0, int(rot_dim), int(pos0),
-                                int(slot0), _ptr(q_out), _stream()))
+    if q is not None and q_out is None:
+        q_out = _rows_like(q, S, H, D)
+    rc = lib().bg_qkv_prologue(cache._h, li, _ptr(q), int(q_stride or D), _ptr(k), _ptr(v), S, H,
+                               _ptr(q_gamma), _ptr(k_gamma), float(eps), _ptr(cos_tab), _ptr(sin_tab),
+                               cos_tab.shape[0] if cos_tab is not None else 0, int(rot_dim), int(pos0),
+                               int(slot0), _ptr(q_out), _stream())
+    if rc:
+        check(rc)
     return q_out
 
 
@@ -384,12 +415,13 @@ def hybrid_full_attention(cache: KvCache, li: int, qg, k, v, S: int, H: int, pos
     D = cache.head_dim
     qr = qkv_prologue(cache, li, qg, k, v, S, H, q_norm, k_norm, eps, cos_tab, sin_tab, rot_dim, pos_base,
                       pos_base, q_stride=2 * D)
-    import torch
     scale = float(np.float32(1.0 / math.sqrt(D)))  # the hybrid's ['f', 1/Math.sqrt(Dh)] param
-    out = torch.empty((S, H, D), dtype=torch.float32, device=qg.device)
+    out = torch.empty_like(qr)
     # the gate half of each [2D] row starts D floats in; its row stride is 2D
-    check(lib().bg_attention(cache.handle, li, _ptr(qr), S, H, int(pos_base), scale,
-                             C.c_void_p(qg.data_ptr() + D * 4), 2 * D, _ptr(out), _stream()))
+    rc = lib().bg_attention(cache._h, li, qr.data_ptr(), S, H, int(pos_base), scale, qg.data_ptr() + D * 4, 2 * D,
+                            out.data_ptr(), _stream())
+    if rc:
+        check(rc)
     return out
 
 
@@ -402,7 +434,6 @@ class OneBitWeight:
     ranges N0 | N1 | N2 for the fused qkv / gate-up weights (src/engine.ts:850-853)."""
 
     def __init__(self, sign, scales, K: int, N0: int, N1: int = 0, N2: int = 0):
-        import torch
         if sign.dtype != torch.int32 or scales.dtype != torch.float32:
             raise TypeError("bitgpu_amd: sign must be int32 (raw u32 words) and scales float32")
         if K % 128 or sign.numel() != (N0 + N1 + N2) * K // 32 or scales.numel() != (N0 + N1 + N2) * K // 128:
@@ -419,18 +450,21 @@ def fused_mm(w: OneBitWeight, x, outs):
     three outputs by range."""
     _f32(x, "x")
     o = list(outs) + [None] * (3 - len(outs))
-    check(lib().bg_gemv_split(_ptr(x), w.K, _ptr(w.sign), _ptr(w.scales), w.N0, w.N1, w.N2, _ptr(o[0]), _ptr(o[1]),
-                              _ptr(o[2]), _stream()))
+    rc = lib().bg_gemv_split(_ptr(x), w.K, _ptr(w.sign), _ptr(w.scales), w.N0, w.N1, w.N2, _ptr(o[0]), _ptr(o[1]),
+                             _ptr(o[2]), _stream())
+    if rc:
+        check(rc)
 
 
 def resid_mm(w: OneBitWeight, x, resid, out=None):
     """residMM at S = 1 (src/engine.ts:1364-1369, matmul_resid_mr_sg.wgsl): W x + resid."""
-    import torch
     _f32(x, "x")
     _f32(resid, "resid")
     if out is None:
-        out = torch.empty(w.N, dtype=torch.float32, device=x.device)
-    check(lib().bg_gemv_resid(_ptr(x), w.K, _ptr(w.sign), _ptr(w.scales), w.N, _ptr(resid), _ptr(out), _stream()))
+        out = x.new_empty(w.N)
+    rc = lib().bg_gemv_resid(_ptr(x), w.K, _ptr(w.sign), _ptr(w.scales), w.N, _ptr(resid), _ptr(out), _stream())
+    if rc:
+        check(rc)
     return out
 
 
@@ -439,17 +473,17 @@ def qkv_proj_prologue(cache: KvCache, li: int, x, w_qkv: OneBitWeight, H: int, q
     """The fused decode branch of ``layer()`` up to the attention (src/engine.ts:1526-1540): the
     qkv projection of the normed hidden state x with Q norm + rope into q_out, K norm + rope into
     the cache and V appended, in one launch. Returns q_out [1, H, D]."""
-    import torch
     D = cache.head_dim
     if w_qkv.N0 != H * D or w_qkv.N1 != cache.kv_heads * D or w_qkv.N2 != cache.kv_heads * D:
         raise ValueError("bitgpu_amd: the qkv weight's row ranges must be H*D | KV*D | KV*D")
     _f32(x, "x")
     if q_out is None:
-        q_out = torch.empty((1, H, D), dtype=torch.float32, device=x.device)
-    check(lib().bg_qkv_proj_prologue(cache.handle, li, _ptr(x), w_qkv.K, _ptr(w_qkv.sign), _ptr(w_qkv.scales), H,
-                                     _ptr(q_norm), _ptr(k_norm), float(eps), _ptr(cos_tab), _ptr(sin_tab),
-                                     int(cos_tab.shape[0]), int(rot_dim), int(pos), int(slot), _ptr(q_out),
-                                     _stream()))
+        q_out = x.new_empty((1, H, D))
+    rc = lib().bg_qkv_proj_prologue(cache._h, li, _ptr(x), w_qkv.K, _ptr(w_qkv.sign), _ptr(w_qkv.scales), H,
+                                    _ptr(q_norm), _ptr(k_norm), float(eps), _ptr(cos_tab), _ptr(sin_tab),
+                                    cos_tab.shape[0], int(rot_dim), int(pos), int(slot), _ptr(q_out), _stream())
+    if rc:
+        check(rc)
     return q_out
 
 
