@@ -65,6 +65,8 @@ SIGNATURES = [
     ("bg_kv_region_bytes", _i32, [_vp, _i32, _i32, C.POINTER(C.c_size_t)]),
     ("bg_kv_export_rows", _i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     ("bg_kv_import_rows", _i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
+    ("bg_kv_save", _i32, [_vp, _i32, _i32, _vp, C.c_size_t, _vp]),
+    ("bg_kv_load", _i32, [_vp, _i32, _i32, _vp, C.c_size_t, _vp]),
 ]
 
 

@@ -8,10 +8,13 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <mutex>
 #include <set>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -156,6 +159,8 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t value, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     p[i] = value;
 }
+
+void drop_snapshot_ring();  // the pinned staging of whole snapshots
 
 // live caches, for bg_stream_sync's check of their merge error words
 std::mutex g_caches_mu;
@@ -473,11 +478,14 @@ int32_t bg_kv_create(int32_t n_layers, int32_t kv_heads, int32_t head_dim, int32
 
 int32_t bg_kv_destroy(bg_kv_cache* c) {
   if (!c) return BG_OK;
+  bool last;
   {
     std::lock_guard<std::mutex> lock(g_caches_mu);
     g_caches.erase(c);
+    last = g_caches.empty();
   }
   (void)hipDeviceSynchronize();
+  if (last) drop_snapshot_ring();
   if (c->err_host) (void)hipHostFree(c->err_host);
   if (c->stage) (void)hipFree(c->stage);
   if (c->proj_raw) (void)hipFree(c->proj_raw);
@@ -1144,6 +1152,196 @@ int32_t bg_kv_import_rows(bg_kv_cache* c, int32_t layer, int32_t region, int32_t
                           void* stream) {
   if (!c) return fail(BG_E_INVALID, "bg_kv_import_rows: NULL cache");
   return transfer(c, layer, region, base, count, const_cast<void*>(host), true, stream);
+}
+
+}  // extern "C"
+
+// ---- whole snapshots ---------------------------------------------------------------------------
+// A snapshot's bytes go through a ring of pinned host slots: a kernel writes a slot (or reads it)
+// over the bus, copying threads move it to (from) the caller's memory, so both run at once and the
+// page faults of fresh memory are shared out. One ring per process, behind a lock for the whole
+// transfer; given back when the last cache goes.
+namespace {
+constexpr int kSlots = 8;
+constexpr size_t kSlotBytes = (size_t)2 << 20;
+struct SnapshotRing {
+  std::mutex mu;
+  char* host = nullptr;
+  char* dev = nullptr;
+  hipEvent_t ev[kSlots] = {};
+  int device = -1;  // of the events
+  void drop() {
+    if (host) (void)hipHostFree(host);
+    for (hipEvent_t& e : ev)
+      if (e) {
+        (void)hipEventDestroy(e);
+        e = nullptr;
+      }
+    host = dev = nullptr;
+    device = -1;
+  }
+  hipError_t ensure(int d) {
+    if (host && device == d) return hipSuccess;
+    drop();
+    hipError_t e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable);
+    if (e != hipSuccess) host = nullptr;
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&dev, host, 0);
+    for (hipEvent_t& x : ev)
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+    if (e != hipSuccess) drop();
+    else device = d;
+    return e;
+  }
+};
+SnapshotRing g_ring;
+
+void drop_snapshot_ring() {
+  std::lock_guard<std::mutex> lock(g_ring.mu);
+  g_ring.drop();
+}
+
+// positions [p0, p1) of one layer: a slot's load
+struct SnapshotPiece {
+  int layer, p0, p1;
+};
+
+// Runs n pieces through the slots. issue(i): main thread, enqueues piece i's kernel and records its
+// event; copy(i): any thread, moves piece i between its slot and the caller. Export copies a piece
+// once its event has passed; import copies it first, once the event of the slot's last piece has.
+template <typename Issue, typename Copy>
+hipError_t snapshot_run(int n, bool import_, Issue issue, Copy copy) {
+  std::mutex mu;
+  std::condition_variable cv;
+  int issued = 0;                    // pieces whose event is recorded
+  std::vector<char> copied(n, 0);
+  hipError_t err = hipSuccess;
+  auto wait_event = [&](int i) {
+    const hipError_t e = hipEventSynchronize(g_ring.ev[i % kSlots]);
+    if (e != hipSuccess) {
+      std::lock_guard<std::mutex> l(mu);
+      err = e;
+    }
+  };
+  auto one = [&](int i) {  // piece i's copy, on a copying thread
+    const int after = import_ ? i - kSlots : i;  // whose event must have passed
+    if (after >= 0) {
+      {
+        std::unique_lock<std::mutex> l(mu);
+        cv.wait(l, [&] { return issued > after || err != hipSuccess; });
+        if (err != hipSuccess) return;
+      }
+      wait_event(after);
+    }
+    copy(i);
+    std::lock_guard<std::mutex> l(mu);
+    copied[i] = 1;
+    cv.notify_all();
+  };
+  std::vector<std::thread> threads;
+  const int want = std::min(4, n);
+  int workers = 0;
+  std::atomic<int> next{0};
+  auto work = [&] {
+    for (int i = next.fetch_add(1); i < n; i = next.fetch_add(1)) one(i);
+  };
+  try {
+    threads.reserve(want);
+    for (; workers < want; workers++) threads.emplace_back(work);
+  } catch (...) {
+    // as many as there are; none: the copies run here
+  }
+  for (int i = 0; i < n; i++) {
+    const int need = import_ ? i : i - kSlots;  // the copy that must be done before the kernel
+    if (need >= 0 && threads.empty() && import_) one(i);
+    if (need >= 0) {
+      std::unique_lock<std::mutex> l(mu);
+      cv.wait(l, [&] { return copied[need] || err != hipSuccess; });
+      if (err != hipSuccess) break;
+    }
+    const hipError_t e = issue(i);
+    {
+      std::lock_guard<std::mutex> l(mu);
+      if (e != hipSuccess) err = e;
+      else issued = i + 1;
+      cv.notify_all();
+    }
+    if (e != hipSuccess) break;
+    if (threads.empty() && !import_) one(i);
+  }
+  {
+    std::lock_guard<std::mutex> l(mu);
+    cv.notify_all();
+  }
+  for (std::thread& t : threads) t.join();
+  return err;
+}
+
+int32_t snapshot(bg_kv_cache* c, int32_t base, int32_t count, char* host, size_t bytes, bool import_, void* stream) {
+  const char* who = import_ ? "bg_kv_load" : "bg_kv_save";
+  if (!c) return fail(BG_E_INVALID, "%s: NULL cache", who);
+  if (count < 0 || base < 0 || (long)base + count > addressable(c))
+    return fail(BG_E_INVALID, "%s: positions %d..%ld beyond capacity %d", who, base, (long)base + count - 1, addressable(c));
+  const size_t per = bg::kv_position_bytes(view(c, 0));  // a position of one layer
+  if (bytes != (size_t)c->n_layers * count * per)
+    return fail(BG_E_INVALID, "%s: %zu bytes for %d layers x %d positions of %zu", who, bytes, c->n_layers, count, per);
+  if (count == 0) return BG_OK;
+  if (!host) return fail(BG_E_INVALID, "%s: NULL host buffer", who);
+  hipStream_t st = (hipStream_t)stream;
+  std::lock_guard<std::mutex> lock(g_ring.mu);
+  hipError_t e = g_ring.ensure(c->device);
+  if (e != hipSuccess) return hip_fail(e, "snapshot staging allocation");
+  std::vector<SnapshotPiece> pieces;
+  const int step = (int)std::max<size_t>(1, kSlotBytes / per);
+  for (int l = 0; l < c->n_layers; l++)
+    for (int p = 0; p < count; p += step) pieces.push_back({l, p, std::min(p + step, count)});
+  if (per > kSlotBytes) return fail(BG_E_UNSUPPORTED, "%s: a position takes %zu bytes", who, per);
+  // a layer's regions, bytes a position, in the snapshot's order
+  const size_t kb = (size_t)c->kv_heads * c->D * elem_bytes(c->dtype);
+  const size_t sb = c->dtype == BG_KV_Q8 ? (size_t)c->kv_heads * (c->D / 32) * sizeof(float) : 0;
+  const size_t region[4] = {kb, kb, sb, sb};
+  e = snapshot_run(
+      (int)pieces.size(), import_,
+      [&](int i) {
+        const SnapshotPiece& q = pieces[i];
+        hipError_t r = bg::launch_kv_stage(view(c, q.layer), base + q.p0, base + q.p1, g_ring.dev + (i % kSlots) * kSlotBytes,
+                                           import_, st);
+        return r == hipSuccess ? hipEventRecord(g_ring.ev[i % kSlots], st) : r;
+      },
+      [&](int i) {
+        const SnapshotPiece& q = pieces[i];
+        char* slot = g_ring.host + (i % kSlots) * kSlotBytes;
+        char* to = host + (size_t)q.layer * count * per;
+        for (int r = 0; r < 4; r++) {
+          const size_t n = (size_t)(q.p1 - q.p0) * region[r];
+          if (import_) memcpy(slot, to + q.p0 * region[r], n);
+          else memcpy(to + q.p0 * region[r], slot, n);
+          slot += n;
+          to += (size_t)count * region[r];
+        }
+      });
+  // (also after an error: nothing may use the slots once the lock is gone)
+  const hipError_t e2 = st ? hipStreamSynchronize(st) : hipDeviceSynchronize();
+  if (e == hipSuccess) e = e2;
+  return e == hipSuccess ? BG_OK : hip_fail(e, import_ ? "snapshot restore" : "snapshot save");
+}
+}  // namespace
+
+extern "C" {
+
+int32_t bg_kv_save(bg_kv_cache* c, int32_t base, int32_t count, void* host, size_t bytes, void* stream) {
+  try {
+    return snapshot(c, base, count, (char*)host, bytes, false, stream);
+  } catch (const std::exception& e) {
+    return fail(BG_E_DEVICE, "bg_kv_save: %s", e.what());
+  }
+}
+
+int32_t bg_kv_load(bg_kv_cache* c, int32_t base, int32_t count, const void* host, size_t bytes, void* stream) {
+  try {
+    return snapshot(c, base, count, (char*)const_cast<void*>(host), bytes, true, stream);
+  } catch (const std::exception& e) {
+    return fail(BG_E_DEVICE, "bg_kv_load: %s", e.what());
+  }
 }
 
 }  // extern "C"

@@ -35,6 +35,10 @@ hipError_t launch_kv_write(const LayerView& L, int which, const float* src, int 
                            hipStream_t st);
 hipError_t launch_kv_export(const LayerView& L, int region, int base, int count, void* dst, hipStream_t st);
 hipError_t launch_kv_import(const LayerView& L, int region, int base, int count, const void* src, hipStream_t st);
+// logical positions [p0, p1) of a layer to or from buf (pinned host memory): K rows, V rows, q8 K
+// and V scales, each region in reference order, kv_position_bytes a position in all
+size_t kv_position_bytes(const LayerView& L);
+hipError_t launch_kv_stage(const LayerView& L, int p0, int p1, void* buf, bool import_, hipStream_t st);
 // f16 copy of slots [0, n_slots) (n_slots a multiple of 32) of a q8 or sink-mode layer, laid out
 // like an f16 cache of the same capacity, with the prefill staging's exact values: q8 dequantized,
 // sink-mode keys rotated at their slot's position. An f16 layer's V is not copied (vdst unused).

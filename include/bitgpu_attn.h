@@ -302,6 +302,13 @@ int32_t bg_kv_export_rows(bg_kv_cache* cache, int32_t layer, int32_t region, int
 int32_t bg_kv_import_rows(bg_kv_cache* cache, int32_t layer, int32_t region, int32_t base,
                           int32_t count, const void* host, void* stream);
 
+/* A whole snapshot's KV bytes at once, the same layout (per layer the K, V and q8 KSCALE, VSCALE
+ * regions of positions base .. base+count-1; src/engine.ts:2757-2771, 2847-2860): `bytes` must be
+ * their sum over layers. Through 16 MiB of pinned staging, shared by the process's caches, kept
+ * until the last one is destroyed; transfers of different caches take turns. Synchronous. */
+int32_t bg_kv_save(bg_kv_cache* cache, int32_t base, int32_t count, void* host, size_t bytes, void* stream);
+int32_t bg_kv_load(bg_kv_cache* cache, int32_t base, int32_t count, const void* host, size_t bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
