@@ -3,8 +3,8 @@
 //
 // Replaces rmsnorm_rope_sg{,_kv16,_kv8}.wgsl (decode), rmsnorm_sg + rope + copy* (prefill) and
 // split_head + rmsnorm + rope_partial + copy* (hybrid) of the reference (src/engine.ts:1527-1540,
-// 1569-1576, 1470-1485). Workgroups of 4 waves, one work item per wave:
-//   Q / K rows 8 (D=128) or 4 (D=256) rows per wave: a lane owns 4 consecutive dims (one
+// 1569-1576, 1470-1485). One work item per wave:
+//   Q / K rows 2 to 8 (D=128) or 1 to 4 (D=256) rows per wave: a lane owns 4 consecutive dims (one
 //              16-byte load), a row spans D/4 lanes; every load (rows and the lanes' cos/sin
 //              entries) is issued before any compute; the sum of squares is a reduction over
 //              the row's lanes (DPP / permlane), and the rotate_half partner (d +- rot/2) comes
@@ -113,29 +113,32 @@ __device__ inline void ld_stream(const float* p, float (&v)[EPL]) {
   }
 }
 
-template <int D>
+template <int D, int NI>
 struct RowLayout {
   static constexpr int LPR = D / 4;         // lanes per row
   static constexpr int RPI = 64 / LPR;      // rows per wave instruction
-  static constexpr int NI = 4;              // load instructions per item
-  static constexpr int RB = RPI * NI;       // rows per wave item
+  static constexpr int RB = RPI * NI;       // rows per wave item of NI load instructions
 };
 
 // SP: every batch of RB rows shares one position (H and KV multiples of RB), so a wave loads one
 // cos/sin row and holds it once (fewer registers: 8 waves a SIMD instead of 6)
-template <int D, int DT, bool SP>
-__global__ __launch_bounds__(256) void qkv_prologue_kernel(LayerView L, PrologueArgs a, PrologueGrid gr) {
-  using RL = RowLayout<D>;
+// NI row load instructions a wave. 4: workgroups of four waves, the items' kinds interleaved; 1 and 2:
+// a wave a workgroup, items in plain order (the interleaving costs five 64-bit divisions, longer
+// than a decode step's rows take to load). Which: prologue_ni.
+template <int D, int DT, bool SP, int NI>
+__global__ __launch_bounds__(NI == 4 ? 256 : 64) void qkv_prologue_kernel(LayerView L, PrologueArgs a, PrologueGrid gr) {
+  using RL = RowLayout<D, NI>;
+  constexpr bool MIX = NI == 4;
   constexpr int EPL = D / 64;
-  constexpr int LPR = RL::LPR, RPI = RL::RPI, NI = RL::NI, RB = RL::RB;
+  constexpr int LPR = RL::LPR, RPI = RL::RPI, RB = RL::RB;
   // each wave's rows for the rotate_half partner (any rot_dim: the partner d +- rot/2 may sit in
   // another lane or straddle lanes)
-  __shared__ __align__(16) float rowbuf[4][RB][D];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ __align__(16) float rowbuf[MIX ? 4 : 1][RB][D];
+  const int wave = MIX ? threadIdx.x >> 6 : 0, lane = threadIdx.x & 63;
   const int KV = L.kv_heads;
   const int d0 = lane * EPL;
 
-  // Work items: Q/K row batches (Q rows first, then K rows) and V items. The kinds are
+  // Work items: Q/K row batches (Q rows first, then K rows) and V items. With MIX the kinds are
   // interleaved evenly over the grid (the V items among all, then the K batches among the Q
   // batches), so the memory-bound Q batches overlap the divide-heavy q8 K rows and the V stores
   // instead of running one after the other.
@@ -143,10 +146,10 @@ __global__ __launch_bounds__(256) void qkv_prologue_kernel(LayerView L, Prologue
   const int nqk_items = (nqk + RB - 1) / RB;
   const int nv_items = (gr.nvs + gr.ng) * KV;
   const long n_items = (long)nqk_items + nv_items;
-  const long pos = (long)blockIdx.x * 4 + wave;
+  const long pos = MIX ? (long)blockIdx.x * 4 + wave : (long)blockIdx.x;
   if (pos >= n_items) return;
-  int item;
-  {
+  int item = (int)pos;
+  if constexpr (MIX) {
     const long v0 = pos * nv_items / n_items, v1 = (pos + 1) * nv_items / n_items;
     if (v1 > v0) {
       item = nqk_items + (int)v0;
@@ -291,6 +294,29 @@ __global__ __launch_bounds__(256) void qkv_prologue_kernel(LayerView L, Prologue
   }
 }
 
+// Load instructions of rows a wave. Few rows are bound by latency and spread over the most waves (a
+// decode step, 32 + 8 heads: 3.1 us, two 3.8, four 5.1; 64 positions 3.9, 4.5, 5.5). Many rows of
+// f16 or q8 keys are best two at a time in plain order (us for 2048 positions f16 / 4096 q8 / 8192
+// q8 at head_dim 256: 18.1 / 36.2 / 83.8, one 19.0 / 37.6 / 91, four interleaved 20.3 / 38.7 / 90);
+// f32 storage, whose V groups write twice the bytes, four interleaved (4096 positions 34.9, in
+// plain order 40; 1500 20.0 against 18.6 with one). The lines lie between the sizes measured: f16
+// and q8 2,560 rows (one) and 13,320 (8.0, two 7.3), f32 60,000 (one) and 98,000.
+static int prologue_ni(int dtype, long rows) {
+  if (rows <= (dtype == KV_F32 ? 65536 : 8192)) return 1;
+  return dtype == KV_F32 ? 4 : 2;
+}
+
+template <int D, int DT, int NI>
+static void launch_prologue(const LayerView& L, const PrologueArgs& a, const PrologueGrid& gr, hipStream_t st) {
+  constexpr int RB = RowLayout<D, NI>::RB, WPB = NI == 4 ? 4 : 1;
+  const long items = ((long)gr.nq + gr.nk + RB - 1) / RB + (long)(gr.nvs + gr.ng) * L.kv_heads;  // one a wave
+  if (items == 0) return;
+  const bool sp = (gr.nq == 0 || a.H % RB == 0) && (gr.nk == 0 || L.kv_heads % RB == 0);
+  const dim3 g((unsigned)((items + WPB - 1) / WPB)), b(64 * WPB);
+  if (sp) hipLaunchKernelGGL((qkv_prologue_kernel<D, DT, true, NI>), g, b, 0, st, L, a, gr);
+  else hipLaunchKernelGGL((qkv_prologue_kernel<D, DT, false, NI>), g, b, 0, st, L, a, gr);
+}
+
 template <int D>
 static hipError_t prologue_d(const LayerView& L, const PrologueArgs& a, hipStream_t st) {
   PrologueGrid gr;
@@ -314,24 +340,19 @@ static hipError_t prologue_d(const LayerView& L, const PrologueArgs& a, hipStrea
     }
     gr.nvs = a.S - 16 * gr.ng;
   }
-  const long items = ((long)gr.nq + gr.nk + RowLayout<D>::RB - 1) / RowLayout<D>::RB + (long)(gr.nvs + gr.ng) * L.kv_heads;
-  if (items == 0) return hipSuccess;
-  dim3 g((unsigned)((items + 3) / 4)), b(256);  // one item per wave
-  constexpr int RB = RowLayout<D>::RB;
-  const bool sp = (gr.nq == 0 || a.H % RB == 0) && (gr.nk == 0 || L.kv_heads % RB == 0);
+  const bool few = prologue_ni(L.dtype, (long)gr.nq + gr.nk) == 1;
   switch (L.dtype) {
     case KV_F32:
-      if (sp) hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_F32, true>), g, b, 0, st, L, a, gr);
-      else hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_F32, false>), g, b, 0, st, L, a, gr);
+      if (few) launch_prologue<D, KV_F32, 1>(L, a, gr, st);
+      else launch_prologue<D, KV_F32, 4>(L, a, gr, st);
       break;
     case KV_F16:
-      if (sp) hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_F16, true>), g, b, 0, st, L, a, gr);
-      else hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_F16, false>), g, b, 0, st, L, a, gr);
+      if (few) launch_prologue<D, KV_F16, 1>(L, a, gr, st);
+      else launch_prologue<D, KV_F16, 2>(L, a, gr, st);
       break;
     default:
-      if (sp) hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_Q8, true>), g, b, 0, st, L, a, gr);
-      else hipLaunchKernelGGL((qkv_prologue_kernel<D, KV_Q8, false>), g, b, 0, st, L, a, gr);
-      break;
+      if (few) launch_prologue<D, KV_Q8, 1>(L, a, gr, st);
+      else launch_prologue<D, KV_Q8, 2>(L, a, gr, st);
   }
   return hipGetLastError();
 }
