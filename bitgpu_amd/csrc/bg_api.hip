@@ -748,7 +748,7 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
 int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
   if (!c || S < 1 || H < 1 || H % c->kv_heads) return fail(BG_E_INVALID, "bg_attention_reserve: bad arguments");
   if (c->dtype == BG_KV_F32 && !bg::f32_split_supported(view(c, 0), S, H)) {
-    if (!ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
+    if (c->D == 128 && !ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
       return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
     return BG_OK;
   }
@@ -1183,7 +1183,7 @@ struct SnapshotRing {
   hipError_t ensure(int d) {
     if (host && device == d) return hipSuccess;
     drop();
-    hipError_t e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable);
+    hipError_t e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
     if (e != hipSuccess) host = nullptr;
     if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&dev, host, 0);
     for (hipEvent_t& x : ev)

@@ -598,7 +598,8 @@ static F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus)
     if (QB < 1) continue;
     const int items = (S + QB - 1) / QB * L.kv_heads;
     auto item = [&](float s) { return 3.8f * (ks == 1 ? 2 * s : 2 * s / ks + 0.4f) + (ks == 1 ? 2.5f : 4.0f); };
-    const int most = std::min(std::min(std::max(1, steps / 2), kPfMaxParts), (int)(kPfSplitBytes / ((size_t)items * rg * 16384)));
+    // (beyond four rounds of the CUs nothing is left to fill)
+    const int most = std::min(std::min(std::max(1, steps / 2), 4 * cus / items), (int)(kPfSplitBytes / ((size_t)items * rg * 16384)));
     for (int np = 1; np <= std::max(1, most) && (np == 1 || (size_t)items * rg * np * 512 <= kPfSplitMlBytes); np++) {
       const int ps = (steps + np - 1) / np;
       if ((steps + ps - 1) / ps != np) continue;
