@@ -86,8 +86,8 @@ struct GemvStep {
 };
 
 // x first: it is needed first, and vector-memory waits retire in issue order. Every load is
-// unconditional (clamped to the last block; past the end x and the scales are zeroed at their use,
-// since a change here would wait for the loads).
+// unconditional (clamped to the last block; past the end x is scaled to 0 and the sum left out at
+// its use, since a change here would wait for the loads).
 template <int T>
 __device__ __forceinline__ void gemv_load(GemvStep<T>& S, const float* __restrict__ x, int K,
                                           const uint32_t* __restrict__ sign, const float* __restrict__ scales, int n0,
@@ -152,8 +152,9 @@ __device__ __forceinline__ void gemv_prepare(GemvX& X, const GemvStep<T>& S, int
   const int e = (int)(mb >> 23) - 126;  // |x| < 2^e
   X.exp = e - 33;
   // weights whose sign bit is masked at bit 4 + j carry 2^(4 + j): x x 2^(27 - e) x 2^(3 - j),
-  // at most 2^30; bit 7 reads as -128. Past the row's end everything becomes 0. (An infinity or
-  // NaN leaves some integer: only its own block sees it, and that one is summed again in f32.)
+  // at most 2^30; bit 7 reads as -128. An infinity or NaN leaves some integer, which only its own
+  // block's sum sees: inside the row that block is summed again in f32; a lane past the row's end
+  // (it holds the last block again) scales finite values to 0, and its sum is never used.
   const int jp = 2 * (l & 1);
   const int h = 1 - ((l >> 1) & 1);
   uint32_t y[2][4];
@@ -249,7 +250,7 @@ __device__ __forceinline__ void gemv_accumulate(float (&acc)[T], const GemvStep<
       if (X.bad) s[t] = gemv_block_f32(x + 128 * b, S.word[t]);
   }
 #pragma unroll
-  for (int t = 0; t < T; t++) acc[t] = fmaf(s[t], X.in ? S.sc[t] : 0.0f, acc[t]);
+  for (int t = 0; t < T; t++) acc[t] = X.in ? fmaf(s[t], S.sc[t], acc[t]) : acc[t];
 }
 
 // One wave's part of the workgroup's rows n0 .. n0 + 16 T - 1: the sums over its steps into

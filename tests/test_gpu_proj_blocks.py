@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from bitgpu_amd import engine as E
-from tests.gpu_helpers import t
+from tests.gpu_helpers import export_k_v, rope_dev, t
 from tests.test_gpu_proj import _check_gemv, _dev_weight, _weight
 
 pytestmark = pytest.mark.gpu
@@ -62,3 +62,35 @@ def test_block_sums_infinities_and_nan(dev):
         got = _run(sign, sc, x, h)
         assert np.array_equal(np.isnan(got), np.isnan(want)) and not np.isfinite(got).any()
         assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
+
+
+@pytest.mark.parametrize("K,N", [(128, 40), (384, 16), (640, 8209), (4224, 40), (8320, 40), (16512, 40)])
+@pytest.mark.parametrize("v", [np.inf, -np.inf])
+def test_infinity_in_the_last_block(dev, K, N, v):
+    """K / 128 no multiple of 4: the last 512-weight step has lanes past the row's end, which load the
+    last block again. An infinity there gives the row's own infinity, not NaN."""
+    rng = np.random.default_rng(K + N)
+    sign, sc = _weight(rng, N, K)
+    x, h = (rng.standard_normal(n).astype(np.float32) for n in (K, N))
+    x[K - 3] = v
+    bit = (sign[:, (K - 3) // 32] >> ((K - 3) % 32)) & 1
+    assert np.array_equal(_run(sign, sc, x, h), np.where(bit, v, -v).astype(np.float32))
+
+
+def test_infinity_in_the_last_block_fused(dev):
+    """The same through the fused qkv projection, on the values it appends (keys and queries are
+    normalized, so there the infinity is NaN by the norm)."""
+    H, KV, D, K, pos = 16, 4, 128, 640, 5
+    rng = np.random.default_rng(8)
+    sign, sc = _weight(rng, (H + 2 * KV) * D, K)
+    x = rng.standard_normal(K).astype(np.float32)
+    x[K - 1] = np.inf
+    cos, sin, _, _ = rope_dev(1e6, D, 64)
+    c = E.KvCache(1, KV, D, "f32", max_seq_len=64, capacity=64)
+    g = t(np.ones(D, np.float32))
+    E.qkv_proj_prologue(c, 0, t(x), _dev_weight(sign, sc, K, H * D, KV * D, KV * D), H, g, g, 1e-6, cos, sin, D, pos, pos)
+    torch.cuda.synchronize()
+    _, v, _, _ = export_k_v(c, 0, pos, 1)
+    bit = sign[(H + KV) * D:, -1] >> 31
+    assert np.array_equal(v.ravel(), np.where(bit, np.inf, -np.inf).astype(np.float32))
+    c.close()
