@@ -103,6 +103,17 @@ def _uninitialized_bytes(n: int) -> bytes:
 _HUGE = 2 << 20
 
 
+def _host_bytes(data):
+    """data as a u8 array: over its own memory where it is a contiguous buffer of single bytes, else
+    over bytes(data). Its size counts bytes (a wider array's len() counts elements)."""
+    try:
+        view = memoryview(data)
+        own = view.c_contiguous and view.itemsize == 1
+    except TypeError:
+        own = False
+    return np.frombuffer(data if own else bytes(data), np.uint8)
+
+
 def rope_tables(theta: float, rot_dim: int, positions: int, yarn: dict | None = None):
     """synthRope (src/engine.ts:117-147): f32 ``[positions, rot_dim/2]`` cos/sin host arrays."""
     half = rot_dim // 2
@@ -313,10 +324,12 @@ class KvCache:
         expect = self.n_layers * sum(self.region_bytes(r, count) for r in self._regions())
         if len(data) != expect:
             raise ValueError(f"restoreCache: snapshot data is {len(data)} bytes, expected {expect}")
+        src = _host_bytes(data)
+        if src.size != expect:
+            raise ValueError(f"restoreCache: snapshot data is {src.size} bytes, expected {expect}")
         self.ensure_capacity(length)
         if expect == 0:
             return
-        src = np.frombuffer(data, np.uint8)
         check(lib().bg_kv_load(self._h, int(base), int(count), src.ctypes.data, expect, _stream()))
 
 

@@ -280,3 +280,40 @@ def test_gemv_argument_validation():
     assert lib.bg_gemv_split(p, 128, p, p, 1, 2, 0, p, None, None, None) == _lib.BG_E_INVALID    # out1 missing
     assert lib.bg_gemv_resid(p, 128, p, p, 4, None, p, None) == _lib.BG_E_INVALID
     assert lib.bg_qkv_proj_prologue(None, 0, p, 128, p, p, 8, p, p, 1e-6, p, p, 8, 128, 0, 0, p, None) == _lib.BG_E_INVALID
+
+
+def _restore_into(monkeypatch, n=12):
+    """A cache of n bytes a position whose library notes what bg_kv_load is given."""
+    seen = []
+
+    class Lib:
+        def bg_kv_load(self, h, base, count, host, nbytes, stream):
+            seen.append((base, count, C.string_at(host, nbytes) if host else None))
+            return 0
+    c = E.KvCache.__new__(E.KvCache)
+    c.n_layers, c.kv_cache, c._h = 1, "f16", None
+    monkeypatch.setattr(E, "lib", Lib)
+    monkeypatch.setattr(E, "_stream", lambda: 0)
+    monkeypatch.setattr(E.KvCache, "region_bytes", lambda self, r, count: count * n // 2)
+    monkeypatch.setattr(E.KvCache, "ensure_capacity", lambda self, length: None)
+    monkeypatch.setattr(E.KvCache, "__del__", lambda self: None)
+    return c, seen
+
+
+def test_restore_takes_any_bytes(monkeypatch):
+    c, seen = _restore_into(monkeypatch)
+    want = bytes(range(200, 224))
+    u8 = np.frombuffer(want, np.uint8)
+    for data in (want, bytearray(want), memoryview(want), u8, u8.view(np.int8), np.repeat(u8, 2)[::2],
+                 memoryview(np.repeat(u8, 2))[::2], list(want)):
+        c.restore_snapshot(data, 5, 3)
+        assert seen.pop() == (3, 2, want)
+
+
+def test_restore_refuses_wider_elements_and_sizes(monkeypatch):
+    """24 elements of 4 bytes are not a snapshot of 24 bytes, nor are 6 of them."""
+    c, seen = _restore_into(monkeypatch)
+    for data in (np.zeros(24, np.int32), np.zeros(6, np.int32), bytes(23), np.zeros(24, np.float64)):
+        with pytest.raises(ValueError):
+            c.restore_snapshot(data, 5, 3)
+    assert not seen
