@@ -328,9 +328,7 @@ class KvCache:
         if src.size != expect:
             raise ValueError(f"restoreCache: snapshot data is {src.size} bytes, expected {expect}")
         self.ensure_capacity(length)
-        if expect == 0:
-            return
-        check(lib().bg_kv_load(self._h, int(base), int(count), src.ctypes.data, expect, _stream()))
+        check(lib().bg_kv_load(self._h, int(base), int(count), src.ctypes.data if expect else None, expect, _stream()))
 
 
 def validate_snapshot(snap, *, roll: bool, sinks: int, kv_cache: str, model: dict, max_seq_len: int,

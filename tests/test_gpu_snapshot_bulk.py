@@ -78,3 +78,12 @@ def test_save_arguments(dev):
     assert c.save_snapshot(0) == b""
     c.restore_snapshot(b"", 0)
     c.close()
+
+
+def test_restore_of_nothing_past_the_cache_is_refused(dev):
+    c = _filled("q8", 1, 8, 128, 64)
+    c.restore_snapshot(b"", 104, 104)  # the end of the cache
+    with pytest.raises(BitgpuError) as e:
+        c.restore_snapshot(b"", 105, 105)
+    assert e.value.code == BG_E_INVALID
+    c.close()

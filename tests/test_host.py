@@ -317,3 +317,9 @@ def test_restore_refuses_wider_elements_and_sizes(monkeypatch):
         with pytest.raises(ValueError):
             c.restore_snapshot(data, 5, 3)
     assert not seen
+
+
+def test_restore_of_nothing_checks_its_range(monkeypatch):
+    c, seen = _restore_into(monkeypatch)
+    c.restore_snapshot(b"", 90, 90)
+    assert seen == [(90, 0, None)]  # the library refuses positions past the capacity
