@@ -10,16 +10,15 @@
 #include <cstring>
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
 #include <mutex>
 #include <set>
 #include <string>
-#include <thread>
 #include <utility>
 #include <vector>
 
 #include "../../include/bitgpu_attn.h"
 #include "bg_kernels.h"
+#include "bg_snapshot.h"
 
 using bg::LayerView;
 
@@ -1155,125 +1154,31 @@ int32_t bg_kv_import_rows(bg_kv_cache* c, int32_t layer, int32_t region, int32_t
 
 }  // extern "C"
 
-// ---- whole snapshots ---------------------------------------------------------------------------
-// A snapshot's bytes go through a ring of pinned host slots: a kernel writes a slot (or reads it)
-// over the bus, copying threads move it to (from) the caller's memory, so both run at once and the
-// page faults of fresh memory are shared out. One ring per process, behind a lock for the whole
-// transfer; given back when the last cache goes.
+// ---- whole snapshots (through the pinned slots of bg_snapshot.h) --------------------------------
 namespace {
-constexpr int kSlots = 8;
-constexpr size_t kSlotBytes = (size_t)2 << 20;
-struct SnapshotRing {
-  std::mutex mu;
-  char* host = nullptr;
-  char* dev = nullptr;
-  hipEvent_t ev[kSlots] = {};
-  int device = -1;  // of the events
-  void drop() {
-    if (host) (void)hipHostFree(host);
-    for (hipEvent_t& e : ev)
-      if (e) {
-        (void)hipEventDestroy(e);
-        e = nullptr;
-      }
-    host = dev = nullptr;
-    device = -1;
-  }
-  hipError_t ensure(int d) {
-    if (host && device == d) return hipSuccess;
-    drop();
-    hipError_t e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
-    if (e != hipSuccess) host = nullptr;
-    if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&dev, host, 0);
-    for (hipEvent_t& x : ev)
-      if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
-    if (e != hipSuccess) drop();
-    else device = d;
-    return e;
-  }
-};
-SnapshotRing g_ring;
+bg::SnapshotRing g_ring;
 
-void drop_snapshot_ring() {
-  std::lock_guard<std::mutex> lock(g_ring.mu);
-  g_ring.drop();
+void drop_snapshot_ring() { g_ring.drop(); }
+
+// a whole snapshot, a call and a staging copy a region
+int32_t snapshot_by_region(bg_kv_cache* c, int32_t base, int32_t count, char* host, bool import_, void* stream) {
+  const int regions = c->dtype == BG_KV_Q8 ? 4 : 2;
+  static constexpr int32_t kOrder[4] = {BG_K, BG_V, BG_KSCALE, BG_VSCALE};
+  for (int l = 0; l < c->n_layers; l++)
+    for (int r = 0; r < regions; r++) {
+      size_t n = 0;
+      int32_t rc = bg_kv_region_bytes(c, kOrder[r], count, &n);
+      if (rc == BG_OK) rc = transfer(c, l, kOrder[r], base, count, host, import_, stream);
+      if (rc != BG_OK) return rc;
+      host += n;
+    }
+  return BG_OK;
 }
 
 // positions [p0, p1) of one layer: a slot's load
 struct SnapshotPiece {
   int layer, p0, p1;
 };
-
-// Runs n pieces through the slots. issue(i): main thread, enqueues piece i's kernel and records its
-// event; copy(i): any thread, moves piece i between its slot and the caller. Export copies a piece
-// once its event has passed; import copies it first, once the event of the slot's last piece has.
-template <typename Issue, typename Copy>
-hipError_t snapshot_run(int n, bool import_, Issue issue, Copy copy) {
-  std::mutex mu;
-  std::condition_variable cv;
-  int issued = 0;                    // pieces whose event is recorded
-  std::vector<char> copied(n, 0);
-  hipError_t err = hipSuccess;
-  auto wait_event = [&](int i) {
-    const hipError_t e = hipEventSynchronize(g_ring.ev[i % kSlots]);
-    if (e != hipSuccess) {
-      std::lock_guard<std::mutex> l(mu);
-      err = e;
-    }
-  };
-  auto one = [&](int i) {  // piece i's copy, on a copying thread
-    const int after = import_ ? i - kSlots : i;  // whose event must have passed
-    if (after >= 0) {
-      {
-        std::unique_lock<std::mutex> l(mu);
-        cv.wait(l, [&] { return issued > after || err != hipSuccess; });
-        if (err != hipSuccess) return;
-      }
-      wait_event(after);
-    }
-    copy(i);
-    std::lock_guard<std::mutex> l(mu);
-    copied[i] = 1;
-    cv.notify_all();
-  };
-  std::vector<std::thread> threads;
-  const int want = std::min(4, n);
-  int workers = 0;
-  std::atomic<int> next{0};
-  auto work = [&] {
-    for (int i = next.fetch_add(1); i < n; i = next.fetch_add(1)) one(i);
-  };
-  try {
-    threads.reserve(want);
-    for (; workers < want; workers++) threads.emplace_back(work);
-  } catch (...) {
-    // as many as there are; none: the copies run here
-  }
-  for (int i = 0; i < n; i++) {
-    const int need = import_ ? i : i - kSlots;  // the copy that must be done before the kernel
-    if (need >= 0 && threads.empty() && import_) one(i);
-    if (need >= 0) {
-      std::unique_lock<std::mutex> l(mu);
-      cv.wait(l, [&] { return copied[need] || err != hipSuccess; });
-      if (err != hipSuccess) break;
-    }
-    const hipError_t e = issue(i);
-    {
-      std::lock_guard<std::mutex> l(mu);
-      if (e != hipSuccess) err = e;
-      else issued = i + 1;
-      cv.notify_all();
-    }
-    if (e != hipSuccess) break;
-    if (threads.empty() && !import_) one(i);
-  }
-  {
-    std::lock_guard<std::mutex> l(mu);
-    cv.notify_all();
-  }
-  for (std::thread& t : threads) t.join();
-  return err;
-}
 
 int32_t snapshot(bg_kv_cache* c, int32_t base, int32_t count, char* host, size_t bytes, bool import_, void* stream) {
   const char* who = import_ ? "bg_kv_load" : "bg_kv_save";
@@ -1286,20 +1191,22 @@ int32_t snapshot(bg_kv_cache* c, int32_t base, int32_t count, char* host, size_t
   if (count == 0) return BG_OK;
   if (!host) return fail(BG_E_INVALID, "%s: NULL host buffer", who);
   hipStream_t st = (hipStream_t)stream;
-  std::lock_guard<std::mutex> lock(g_ring.mu);
-  hipError_t e = g_ring.ensure(c->device);
-  if (e != hipSuccess) return hip_fail(e, "snapshot staging allocation");
+  constexpr int kSlots = bg::SnapshotRing::kSlots;
+  constexpr size_t kSlotBytes = bg::SnapshotRing::kSlotBytes;
+  // a position wider than a slot, the slots in use by another transfer, no pinned memory for them
+  const bool fits = per <= kSlotBytes;
+  std::unique_lock<std::mutex> lock = fits ? g_ring.take(c->device) : std::unique_lock<std::mutex>();
+  if (!lock) return snapshot_by_region(c, base, count, host, import_, stream);
   std::vector<SnapshotPiece> pieces;
-  const int step = (int)std::max<size_t>(1, kSlotBytes / per);
+  const int step = (int)(kSlotBytes / per);
   for (int l = 0; l < c->n_layers; l++)
     for (int p = 0; p < count; p += step) pieces.push_back({l, p, std::min(p + step, count)});
-  if (per > kSlotBytes) return fail(BG_E_UNSUPPORTED, "%s: a position takes %zu bytes", who, per);
   // a layer's regions, bytes a position, in the snapshot's order
   const size_t kb = (size_t)c->kv_heads * c->D * elem_bytes(c->dtype);
   const size_t sb = c->dtype == BG_KV_Q8 ? (size_t)c->kv_heads * (c->D / 32) * sizeof(float) : 0;
   const size_t region[4] = {kb, kb, sb, sb};
-  e = snapshot_run(
-      (int)pieces.size(), import_,
+  hipError_t e = bg::snapshot_run(
+      g_ring, (int)pieces.size(), import_,
       [&](int i) {
         const SnapshotPiece& q = pieces[i];
         hipError_t r = bg::launch_kv_stage(view(c, q.layer), base + q.p0, base + q.p1, g_ring.dev + (i % kSlots) * kSlotBytes,

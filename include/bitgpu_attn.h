@@ -305,7 +305,8 @@ int32_t bg_kv_import_rows(bg_kv_cache* cache, int32_t layer, int32_t region, int
 /* A whole snapshot's KV bytes at once, the same layout (per layer the K, V and q8 KSCALE, VSCALE
  * regions of positions base .. base+count-1; src/engine.ts:2757-2771, 2847-2860): `bytes` must be
  * their sum over layers. Through 16 MiB of pinned staging, shared by the process's caches, kept
- * until the last one is destroyed; transfers of different caches take turns. Synchronous. */
+ * until the last one is destroyed. A transfer that finds it in use by another cache's, cannot have
+ * it, or whose positions exceed a 2 MiB slot goes region by region as above. Synchronous. */
 int32_t bg_kv_save(bg_kv_cache* cache, int32_t base, int32_t count, void* host, size_t bytes, void* stream);
 int32_t bg_kv_load(bg_kv_cache* cache, int32_t base, int32_t count, const void* host, size_t bytes, void* stream);
 

@@ -87,3 +87,15 @@ def test_restore_of_nothing_past_the_cache_is_refused(dev):
         c.restore_snapshot(b"", 105, 105)
     assert e.value.code == BG_E_INVALID
     c.close()
+
+
+def test_positions_wider_than_a_staging_slot(dev):
+    """2,100 kv heads of f32: 2.15 MB a position, past a 2 MiB slot; goes region by region."""
+    a = _filled("f32", 1, 2100, 128, 3)
+    data = a.save_snapshot(3)
+    assert data == _by_region(a, 3)
+    b = _filled("f32", 1, 2100, 128, 3, seed=1)
+    b.restore_snapshot(data, 3)
+    assert _by_region(b, 3) == data
+    a.close()
+    b.close()
