@@ -1195,7 +1195,7 @@ int32_t snapshot(bg_kv_cache* c, int32_t base, int32_t count, char* host, size_t
   constexpr size_t kSlotBytes = bg::SnapshotRing::kSlotBytes;
   // a position wider than a slot, the slots in use by another transfer, no pinned memory for them
   const bool fits = per <= kSlotBytes;
-  std::unique_lock<std::mutex> lock = fits ? g_ring.take(c->device) : std::unique_lock<std::mutex>();
+  std::unique_lock<std::mutex> lock = fits ? g_ring.take() : std::unique_lock<std::mutex>();
   if (!lock) return snapshot_by_region(c, base, count, host, import_, stream);
   std::vector<SnapshotPiece> pieces;
   const int step = (int)(kSlotBytes / per);

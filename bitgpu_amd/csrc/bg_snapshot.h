@@ -25,11 +25,11 @@ struct SnapshotRing {
   hipEvent_t ev[kSlots] = {};
   int device = -1;  // of the events
 
-  // The ring for one transfer, held as long as the lock; an empty lock when another transfer has it
-  // or its slots cannot be had.
-  std::unique_lock<std::mutex> take(int d) {
+  // The ring for one transfer on the current device, held as long as the lock; an empty lock when
+  // another transfer has it or its slots cannot be had.
+  std::unique_lock<std::mutex> take() {
     std::unique_lock<std::mutex> lock(mu, std::try_to_lock);
-    if (lock && ensure(d) != hipSuccess) {
+    if (lock && ensure() != hipSuccess) {
       (void)hipGetLastError();
       lock.unlock();
     }
@@ -42,21 +42,30 @@ struct SnapshotRing {
   }
 
  private:
-  void give_back() {
-    if (host) (void)hipHostFree(host);
+  void drop_events() {
     for (hipEvent_t& e : ev)
       if (e) {
         (void)hipEventDestroy(e);
         e = nullptr;
       }
-    host = dev = nullptr;
     device = -1;
   }
-  hipError_t ensure(int d) {
-    if (host && device == d) return hipSuccess;
-    give_back();
-    hipError_t e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
-    if (e != hipSuccess) host = nullptr;
+  void give_back() {
+    drop_events();
+    if (host) (void)hipHostFree(host);
+    host = dev = nullptr;
+  }
+  // The slots serve every device. Events are the device's that was current at their creation and
+  // can be recorded on its streams alone, so it is that device, not a cache's, they are kept for.
+  hipError_t ensure() {
+    int d = 0;
+    hipError_t e = hipGetDevice(&d);
+    if (e != hipSuccess || (host && device == d)) return e;
+    drop_events();
+    if (!host) {
+      e = hipHostMalloc((void**)&host, kSlots * kSlotBytes, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
+      if (e != hipSuccess) host = nullptr;
+    }
     if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&dev, host, 0);
     for (hipEvent_t& x : ev)
       if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);

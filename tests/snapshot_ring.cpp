@@ -74,7 +74,7 @@ static bool round_trip(int n) {
 
 int main() {
   {
-    auto lock = ring.take(0);
+    auto lock = ring.take();
     CHECK(lock);
     for (int n : {1, 7, 8, 9, 61}) CHECK(round_trip(n));
     // a kernel that cannot be launched ends the transfer with its error
@@ -83,16 +83,23 @@ int main() {
     // the ring is taken: another transfer is told so at once
     bool other = true;
     const auto t0 = std::chrono::steady_clock::now();
-    std::thread([&] { other = (bool)ring.take(0); }).join();
+    std::thread([&] { other = (bool)ring.take(); }).join();
     CHECK(!other && std::chrono::steady_clock::now() - t0 < std::chrono::seconds(5));
   }
-  CHECK(ring.take(0) && g_allocs == 1);
+  CHECK(ring.take() && g_allocs == 1);
+  // another device current: its own events, the same slots, and back
+  for (int d : {1, 1, 0}) {
+    g_device = d;
+    CHECK(ring.take());
+    for (hipEvent_t e : ring.ev) CHECK(((Event*)e)->device == d);
+  }
+  CHECK(g_allocs == 1);
   ring.drop();
   CHECK(g_live == 0);
   g_no_memory = true;
-  CHECK(!ring.take(0) && g_live == 0);
+  CHECK(!ring.take() && g_live == 0);
   g_no_memory = false;
-  CHECK(ring.take(0));
+  CHECK(ring.take());
   ring.drop();
   CHECK(g_live == 0);
   printf("ok\n");
