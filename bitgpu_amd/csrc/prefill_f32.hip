@@ -55,7 +55,7 @@ struct F32PrefillParams {
   const float* gate;
   int gate_stride;
   float* out;
-  int n_scan_fixed;  // sink mode: physical slots scanned by every block; 0: causal bound
+  int n_scan_fixed;  // >0: physical slots scanned by every block (sink mode after a wrap); 0: causal bound
   int phys_limit;
   int n_qblocks;
   int mirror;
@@ -676,7 +676,7 @@ hipError_t launch_attention_f32(const LayerView& L, const AttnArgs& a, hipStream
   p.gate = a.gate;
   p.gate_stride = a.gate_stride;
   p.out = a.out;
-  p.n_scan_fixed = L.ring.roll ? ((L.ring.head != 0) ? L.max_seq : a.pos_base + a.S) : 0;
+  p.n_scan_fixed = (L.ring.roll && L.ring.head != 0) ? L.max_seq : 0;
   p.phys_limit = L.ring.roll ? L.max_seq : L.cap;
   p.n_qblocks = (a.S + p.QB - 1) / p.QB;
   const F32Plan f = f32_plan(L, a.S, a.H, a.pos_base, a.num_cus > 0 ? a.num_cus : 256);

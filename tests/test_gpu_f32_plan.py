@@ -50,3 +50,14 @@ def test_f32_sink_ring(dev, window, moves, fill, S, mode):
     c, q, want = _ring("f32", 32, 8, 128, window, moves, fill, S, mode)
     assert np.abs(run_attention(c, 0, q, fill) - want).max() <= 1e-4
     c.close()
+
+
+@pytest.mark.parametrize("H,KV,D,fill,S,mode", [
+    (32, 8, 128, 0, 333, "slot"), (16, 4, 128, 650, 70, "absolute"), (8, 2, 256, 0, 150, "slot")])
+def test_f32_sink_prompt_before_any_eviction(dev, H, KV, D, fill, S, mode):
+    """The ring's origin has not moved: the causal bound, as for the plain cache."""
+    c, q, want = _ring("f32", H, KV, D, 1000, (), fill, S, mode)
+    out = run_attention(c, 0, q, fill)
+    assert np.abs(out - want).max() <= 1e-4
+    assert np.array_equal(run_attention_noalloc(c, 0, q, fill), out)
+    c.close()
