@@ -34,6 +34,7 @@ SIGNATURES = [
     ("bg_ring_map", _i32, [_i32, _i32, _i32, _i32, _pi32]),
     ("bg_stream_sync", _i32, [_vp]),
     ("bg_decode_plan", _i32, [_i32] * 8 + [_pi32]),
+    ("bg_f32_prefill_plan", _i32, [_i32] * 9 + [_pi32]),
     ("bg_diag_stream_read", _i32, [_vp, C.c_size_t, _i32, _i32, _vp, _vp]),
     ("bg_debug_merge_hooks", _i32, [_i32, _i32]),
     ("bg_stream_create", _i32, [C.POINTER(_vp)]),

@@ -1076,6 +1076,31 @@ int32_t bg_decode_plan(int32_t kv_heads, int32_t head_dim, int32_t dtype, int32_
   return BG_OK;
 }
 
+int32_t bg_f32_prefill_plan(int32_t kv_heads, int32_t S, int32_t H, int32_t pos_base, int32_t window, int32_t sinks,
+                            int32_t head, int32_t num_cus, int32_t partials, int32_t* out) {
+  if (!out || kv_heads < 1 || S < 1 || H < kv_heads || H % kv_heads || pos_base < 0 || num_cus < 1)
+    return fail(BG_E_INVALID, "bg_f32_prefill_plan: bad arguments");
+  if (window && (sinks < 1 || window <= sinks || head < 0 || head >= window - sinks || (long)pos_base + S > window))
+    return fail(BG_E_INVALID, "bg_f32_prefill_plan: ring of %d slots, %d sinks, origin %d", window, sinks, head);
+  LayerView L{};
+  L.kv_heads = kv_heads;
+  L.D = 128;
+  L.dtype = bg::KV_F32;
+  L.max_seq = window ? window : pos_base + S;
+  L.cap = round32(L.max_seq);
+  L.ring.roll = window > 0;
+  L.ring.sinks = window ? sinks : 0;
+  L.ring.W = L.max_seq - L.ring.sinks;
+  L.ring.head = window ? head : 0;
+  const bg::F32Plan p = bg::f32_plan(L, S, H, pos_base, num_cus, partials ? bg::kPfSplitBytes / sizeof(float) : 0);
+  if (!p.QB) return fail(BG_E_UNSUPPORTED, "bg_f32_prefill_plan: no plan for %d heads on %d", H, kv_heads);
+  out[0] = p.ks;
+  out[1] = p.QB;
+  out[2] = p.n_parts;
+  out[3] = p.part_steps;
+  return BG_OK;
+}
+
 int32_t bg_diag_stream_read(const void* buf, size_t bytes, int32_t workgroups, int32_t nontemporal, uint32_t* sink,
                             void* stream) {
   if (!buf || !sink || bytes == 0 || bytes % 16 || workgroups < 1 || workgroups > 65535)

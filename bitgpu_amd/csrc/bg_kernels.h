@@ -169,6 +169,14 @@ hipError_t launch_prefill_merge(const LayerView& L, const AttnArgs& a, int QB, i
                                 int n_scan_fixed, int skip_n, hipStream_t st);
 // the KT-slot steps *t0 .. + *n - 1 of a wrapped ring that hold only slots past S rows at pos_base
 void prefill_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n);
+// The plan of an f32 prefill launch (host-only arithmetic): ks of a workgroup's four waves share 32
+// rows and take every ks-th 32-key step (4 / ks row groups an item), QB queries an item, n_parts
+// parts of part_steps 64-key steps, at most `floats` floats of partials. QB = 0: the kernel of 128-row
+// items staged through LDS (head_dim 256, whose K, V, Q and O a step would not fit a wave's registers).
+struct F32Plan {
+  int ks, QB, n_parts, part_steps;
+};
+F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus, size_t floats);
 // floats of the partials an f32 prefill uses at pos_base (0: none)
 size_t f32_prefill_floats(const LayerView& L, int S, int H, int pos_base, int num_cus);
 bool prefill_can_split(const LayerView& L, int S, int H, int num_cus);

@@ -569,20 +569,15 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_split_kernel(F32SplitParam
   if (sp.n_parts > 1 && ks == 0) sp.pml[pi * 64 + lane] = make_float2(M, lt);
 }
 
-// The plan of a launch: KS waves share a 32-row group's keys, QB queries an item (QB x G rows of
-// 4 / KS row groups), n_parts parts of part_steps 64-key steps; QB = 0: the kernel above (head_dim
-// 256, whose K, V, Q and O a step would not fit a wave's registers).
-struct F32Plan {
-  int ks, QB, n_parts, part_steps;
-};
-
 // The cheapest by a cost model in us. A step takes 3.8 us of a wave (a CU runs one workgroup); an
 // item 2.5 to 4 before and after its steps. Where items are alike (a long context before the rows)
 // the grid runs in whole rounds of the CUs, else its longest item or its share of a CU counts,
 // whichever is more. Keys and values of a kv head past an XCD's L2 are read at about 5 TB/s for
 // every item; a partial (16 KB and (m, l) a row group) is written and read at about 4.5 TB/s and
-// the merge adds 5 us.
-static F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus) {
+// the merge adds 5 us. Without room for a plan's partials (`floats` of them) the cheapest of one part:
+// what is cheapest in many parts is not (200 rows of 16 heads on 4 after 9,000 keys: nine parts of 128
+// rows, but in one part items of 32; captured without a buffer 1,155 -> 303 us).
+F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus, size_t floats) {
   F32Plan best{4, 0, 1, 0};
   const int G = H / L.kv_heads;
   if (L.D != 128 || G > 128) return best;
@@ -599,7 +594,7 @@ static F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus)
     const int items = (S + QB - 1) / QB * L.kv_heads;
     auto item = [&](float s) { return 3.8f * (ks == 1 ? 2 * s : 2 * s / ks + 0.4f) + (ks == 1 ? 2.5f : 4.0f); };
     // (beyond four rounds of the CUs nothing is left to fill)
-    const int most = std::min(std::min(std::max(1, steps / 2), 4 * cus / items), (int)(kPfSplitBytes / ((size_t)items * rg * 16384)));
+    const int most = std::min(std::min(std::max(1, steps / 2), 4 * cus / items), (int)(floats / ((size_t)items * rg * 4096)));
     for (int np = 1; np <= std::max(1, most) && (np == 1 || (size_t)items * rg * np * 512 <= kPfSplitMlBytes); np++) {
       const int ps = (steps + np - 1) / np;
       if ((steps + ps - 1) / ps != np) continue;
@@ -617,7 +612,7 @@ static F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus)
 }
 
 size_t f32_prefill_floats(const LayerView& L, int S, int H, int pos_base, int cus) {
-  const F32Plan f = f32_plan(L, S, H, pos_base, cus);
+  const F32Plan f = f32_plan(L, S, H, pos_base, cus, kPfSplitBytes / sizeof(float));
   return f.QB && f.n_parts > 1 ? (size_t)((S + f.QB - 1) / f.QB) * L.kv_heads * f.n_parts * (4 / f.ks) * 4096 : 0;
 }
 
@@ -679,7 +674,8 @@ hipError_t launch_attention_f32(const LayerView& L, const AttnArgs& a, hipStream
   p.n_scan_fixed = (L.ring.roll && L.ring.head != 0) ? L.max_seq : 0;
   p.phys_limit = L.ring.roll ? L.max_seq : L.cap;
   p.n_qblocks = (a.S + p.QB - 1) / p.QB;
-  const F32Plan f = f32_plan(L, a.S, a.H, a.pos_base, a.num_cus > 0 ? a.num_cus : 256);
+  const size_t room = a.pf_o && a.pf_ml ? std::min(a.pf_floats, kPfSplitBytes / sizeof(float)) : 0;
+  const F32Plan f = f32_plan(L, a.S, a.H, a.pos_base, a.num_cus > 0 ? a.num_cus : 256, room);
   if (f.QB) {
     F32SplitParams sp;
     p.QB = f.QB;
@@ -688,8 +684,6 @@ hipError_t launch_attention_f32(const LayerView& L, const AttnArgs& a, hipStream
     sp.n_parts = f.n_parts;
     sp.part_steps = f.part_steps;
     prefill_skip(L, a.S, a.pos_base, 64, &sp.skip_t0, &sp.skip_n);
-    // (without a buffer for the partials: one part)
-    if (!a.pf_o || !a.pf_ml || (size_t)p.n_qblocks * L.kv_heads * f.n_parts * (4 / f.ks) * 4096 > a.pf_floats) sp.n_parts = 1;
     sp.pws = (float4*)a.pf_o;
     sp.pml = (float2*)a.pf_ml;
     sp.b = p;

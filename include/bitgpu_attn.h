@@ -104,6 +104,13 @@ int32_t bg_stream_sync(void* stream);
 int32_t bg_decode_plan(int32_t kv_heads, int32_t head_dim, int32_t dtype, int32_t S, int32_t H,
                        int32_t pos_base, int32_t num_cus, int32_t resident_per_cu, int32_t* out);
 
+/* The same for the f32 prefill at head_dim 128: out[0..3] = waves of a workgroup (of four) that
+ * share 32 rows, queries per workgroup, parts the key range is split into, 64-key steps per part.
+ * window > 0: a sink-mode ring of that many slots with `sinks` sinks and origin `head`; partials 0:
+ * a launch that has no buffer for split partials. */
+int32_t bg_f32_prefill_plan(int32_t kv_heads, int32_t S, int32_t H, int32_t pos_base, int32_t window,
+                            int32_t sinks, int32_t head, int32_t num_cus, int32_t partials, int32_t* out);
+
 /* Test hook with no counterpart in the reference: the decode split merge's poll bound
  * (spin_limit polls before a merger gives up; 0 = the default, 2^20) and one split index that
  * stores no partial (-1 = none), for every later bg_attention / bg_attention_noalloc call in

@@ -3,9 +3,11 @@ split over workgroups, heads per kv head that do not divide 32, wrapped sink rin
 oracle (max-abs 1e-4, the bar for f32 storage)."""
 import numpy as np
 import pytest
+import torch
 
+from bitgpu_amd import engine as E
 from oracle import ref
-from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc
+from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc, t
 from tests.test_gpu_sink_copy import _ring
 from tests.test_gpu_split_prefill import _case
 
@@ -60,4 +62,26 @@ def test_f32_sink_prompt_before_any_eviction(dev, H, KV, D, fill, S, mode):
     out = run_attention(c, 0, q, fill)
     assert np.abs(out - want).max() <= 1e-4
     assert np.array_equal(run_attention_noalloc(c, 0, q, fill), out)
+    c.close()
+
+
+def test_f32_captured_without_reserve(dev):
+    """No buffer for partials can be had under capture: one part, on the rows planned for that."""
+    H, KV, ctx, S = 16, 4, 9000, 200
+    c, _, q, _ = _case("f32", H, KV, 128, ctx + S, S, seed=4, gate=False)
+    qt, out = t(q), torch.empty(S, H, 128, device="cuda")
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        E.attention(c, 0, qt, S, H, ctx, out=out)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    rows = [0, 7, 8, 31, 32, 100, 199]
+    want = np.concatenate([ref.attention(q[r:r + 1], kk[:ctx + r + 1], vv[:ctx + r + 1], ctx + r) for r in rows])
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert np.isfinite(got).all() and np.abs(got[rows] - want).max() <= 1e-4
     c.close()

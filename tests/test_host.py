@@ -241,6 +241,36 @@ def test_decode_plan_residency_cap():
     assert _plan(8, 128, 64, 32, 1000)[0] == _lib.BG_E_UNSUPPORTED
 
 
+def f32_plan(KV, S, H, pos_base, window=0, sinks=0, head=0, partials=1, cus=256):
+    out = (C.c_int32 * 4)()
+    rc = _lib.lib().bg_f32_prefill_plan(KV, S, H, pos_base, window, sinks, head, cus, partials, out)
+    return rc, list(out)
+
+
+@pytest.mark.parametrize("KV,S,H,pos_base,window,head", [
+    (8, 777, 16, 0, 0, 0), (4, 200, 16, 9000, 0, 0), (8, 9, 32, 5000, 0, 0), (2, 104, 16, 1000, 0, 0),
+    (1, 40, 12, 700, 0, 0), (8, 600, 32, 16000, 0, 0), (4, 83, 24, 1911, 2004, 300), (1, 3, 100, 50, 0, 0)])
+def test_f32_plan_covers_the_keys(KV, S, H, pos_base, window, head):
+    """Four waves as row groups x key shares, a group's rows within 32, parts that cover every step
+    with none empty; without room for partials one part, on the rows that are cheapest in one part."""
+    rc, (ks, QB, np_, ps) = f32_plan(KV, S, H, pos_base, window, 4, head)
+    assert rc == 0 and ks in (1, 2, 4) and 1 <= QB * (H // KV) <= 128 // ks
+    seen, steps = (pos_base + S + 63) // 64, ((window or pos_base + S) + 63) // 64  # a ring's masked steps may be left out
+    assert np_ * ps >= seen and (np_ - 1) * ps < steps
+    rc, one = f32_plan(KV, S, H, pos_base, window, 4, head, partials=0)
+    assert rc == 0 and one[2] == 1
+
+
+def test_f32_plan_without_partials():
+    # 200 rows of 16 heads on 4 after 9,000 keys: nine parts of 128-row items; in one part items of
+    # 32 rows, four times the workgroups and a quarter of the chain
+    assert f32_plan(4, 200, 16, 9000)[1][:3] == [1, 32, 9]
+    assert f32_plan(4, 200, 16, 9000, partials=0)[1][:3] == [4, 8, 1]
+    assert f32_plan(8, 600, 32, 16000)[1][:3] == [1, 32, 3]
+    assert f32_plan(1, 3, 200, 0)[0] == _lib.BG_E_UNSUPPORTED  # more than 128 heads a kv head
+    assert f32_plan(8, 3, 32, 1000, window=1000, sinks=4)[0] == _lib.BG_E_INVALID
+
+
 def test_diag_stream_read_argument_validation():
     lib = _lib.lib()
     buf = (C.c_uint32 * 64)()
