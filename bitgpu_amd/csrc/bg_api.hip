@@ -41,12 +41,9 @@ struct bg_kv_cache {
   size_t ws_counters = 0;
   // f16 copy of one q8 or sink-mode layer's attended slots for long prefills (K then, q8, V)
   void* pf16 = nullptr;
-  // split-K prefill: partials (a larger buffer replaces a smaller one, which is kept until destroy
-  // for the launches captured with it) and their (m, l), bg::kPfSplitMlBytes once allocated
-  float* pf_o = nullptr;
-  size_t pf_floats = 0;
-  float* pf_ml = nullptr;
-  std::vector<float*> retired_pf;
+  // split-K prefill: bg::kPfSplitBytes of partials (as many as any plan uses, so that no launch
+  // captured in a graph is left with a smaller buffer), then their (m, l)
+  float* pf = nullptr;
   // workspaces replaced by a larger one, kept until destroy: launches captured in a graph before
   // the growth still use them (and find their slots holding the empty marker)
   std::vector<std::pair<float*, size_t>> retired_ws;
@@ -492,9 +489,7 @@ int32_t bg_kv_destroy(bg_kv_cache* c) {
   if (c->ws) (void)hipFree(c->ws);
   if (c->ws_count) (void)hipFree(c->ws_count);
   if (c->pf16) (void)hipFree(c->pf16);
-  if (c->pf_o) (void)hipFree(c->pf_o);
-  if (c->pf_ml) (void)hipFree(c->pf_ml);
-  for (float* r : c->retired_pf) (void)hipFree(r);
+  if (c->pf) (void)hipFree(c->pf);
   for (const auto& r : c->retired_ws) (void)hipFree(r.first);
   for (unsigned* r : c->retired_count) (void)hipFree(r);
   delete c;
@@ -687,31 +682,23 @@ static int32_t ensure_workspace_floats(bg_kv_cache* c, size_t need, size_t count
   return BG_OK;
 }
 
-// Split-K prefill: buffers for `floats` floats of partials and their (m, l). False when they cannot
-// be had (out of memory, or the stream is being captured): the launch then scans whole key ranges,
-// which needs none.
-static bool ensure_prefill_split(bg_kv_cache* c, size_t floats, hipStream_t st) {
-  if (floats <= c->pf_floats && c->pf_ml) return true;
+// Split-K prefill: the buffer of partials and their (m, l). False when it cannot be had (out of
+// memory, or the stream is being captured): the launch then scans whole key ranges, which needs none.
+static bool ensure_prefill_split(bg_kv_cache* c, hipStream_t st) {
+  if (c->pf) return true;
   if (capturing(st)) return false;
-  if (floats < 2 * c->pf_floats) floats = 2 * c->pf_floats;  // few buffers are ever retired
-  if (floats > bg::kPfSplitBytes / sizeof(float)) floats = bg::kPfSplitBytes / sizeof(float);
-  float* o = nullptr;
-  float* ml = nullptr;
-  hipError_t e = hipSuccess;
-  if (floats > c->pf_floats) e = hipMalloc((void**)&o, floats * sizeof(float));
-  if (e == hipSuccess && !c->pf_ml) e = hipMalloc((void**)&ml, bg::kPfSplitMlBytes);
-  if (e != hipSuccess) {
+  if (hipMalloc((void**)&c->pf, bg::kPfSplitBytes + bg::kPfSplitMlBytes) != hipSuccess) {
     (void)hipGetLastError();
-    if (o) (void)hipFree(o);
-    return false;
+    c->pf = nullptr;
   }
-  if (o) {
-    if (c->pf_o) c->retired_pf.push_back(c->pf_o);
-    c->pf_o = o;
-    c->pf_floats = floats;
-  }
-  if (ml) c->pf_ml = ml;
-  return true;
+  return c->pf != nullptr;
+}
+
+// a launch's split partials in `pf` (kPfSplitBytes + kPfSplitMlBytes)
+static void use_prefill_split(bg::AttnArgs& a, float* pf) {
+  a.pf_o = pf;
+  a.pf_floats = bg::kPfSplitBytes / sizeof(float);
+  a.pf_ml = pf + a.pf_floats;
 }
 
 static int32_t ensure_workspace(bg_kv_cache* c, int S, int H) {
@@ -747,7 +734,7 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
 int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
   if (!c || S < 1 || H < 1 || H % c->kv_heads) return fail(BG_E_INVALID, "bg_attention_reserve: bad arguments");
   if (c->dtype == BG_KV_F32 && !bg::f32_split_supported(view(c, 0), S, H)) {
-    if (c->D == 128 && !ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
+    if (c->D == 128 && !ensure_prefill_split(c, nullptr))
       return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
     return BG_OK;
   }
@@ -757,7 +744,7 @@ int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
       if (rc != BG_OK) return rc;
     }
     if (bg::prefill_can_split(view(c, 0), S, H, c->num_cus) &&
-        !ensure_prefill_split(c, bg::kPfSplitBytes / sizeof(float), nullptr))
+        !ensure_prefill_split(c, nullptr))
       return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
     return BG_OK;
   }
@@ -833,11 +820,7 @@ int32_t bg_attention(bg_kv_cache* c, int32_t layer, const float* q, int32_t S, i
     e = bg::launch_attention_f32_split(L, a, st);
   } else if (c->dtype == BG_KV_F32) {
     const size_t pf = bg::f32_prefill_floats(L, S, H, pos_base, c->num_cus);
-    if (pf > 0 && ensure_prefill_split(c, pf, st)) {
-      a.pf_o = c->pf_o;
-      a.pf_ml = c->pf_ml;
-      a.pf_floats = c->pf_floats;
-    }
+    if (pf > 0 && ensure_prefill_split(c, st)) use_prefill_split(a, c->pf);
     e = bg::launch_attention_f32(L, a, st);
   } else if (bg::decode_preferred(L, S, H)) {
     int32_t rc = ensure_workspace(c, S, H);
@@ -848,11 +831,7 @@ int32_t bg_attention(bg_kv_cache* c, int32_t layer, const float* q, int32_t S, i
     e = bg::launch_attention_decode(L, a, st);
   } else if (bg::prefill_supported(L, S, H)) {
     const size_t pf = bg::prefill_workspace_floats(L, S, H, pos_base, c->num_cus);
-    if (pf > 0 && ensure_prefill_split(c, pf, st)) {
-      a.pf_o = c->pf_o;
-      a.pf_ml = c->pf_ml;
-      a.pf_floats = c->pf_floats;
-    }
+    if (pf > 0 && ensure_prefill_split(c, st)) use_prefill_split(a, c->pf);
     bool copy = bg::prefill_wants_f16_copy(L, S, H);
     if (copy && !(c->pf16 && c->pf16_cap == c->cap)) {
       // sink mode can rotate at staging instead (the same values), where the copy cannot be had
@@ -924,9 +903,7 @@ int32_t bg_attention_noalloc(bg_kv_cache* c, int32_t layer, const float* q, int3
   LayerView L = view(c, layer);
   bg::AttnArgs a = attention_args(c, q, S, H, pos_base, scale, gate, gate_stride, out);
   // a prefill that splits its key ranges keeps its partials in the scratch, which holds every plan's
-  a.pf_o = (float*)((char*)ptr + kScratchBytes);
-  a.pf_floats = bg::kPfSplitBytes / sizeof(float);
-  a.pf_ml = (float*)((char*)ptr + kScratchBytes + bg::kPfSplitBytes);
+  use_prefill_split(a, (float*)((char*)ptr + kScratchBytes));
   if (c->dtype == BG_KV_F32) {
     // the matrix-core kernel for every shape
     e = bg::launch_attention_f32(L, a, st);

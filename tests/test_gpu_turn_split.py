@@ -47,3 +47,20 @@ def test_turn_captured_without_reserve(dev):
         torch.cuda.synchronize()
         _check(out.cpu().numpy(), want)
     c.close()
+
+
+def test_split_partials_stay_within_their_bound(dev):
+    """Plans of growing partials use one buffer of 33 MiB, as the header states (the memory in use
+    grows by no more, rounded up to the allocator's pages)."""
+    H, KV, D, ctx = 32, 8, 128, 16000
+    q, out = torch.randn(333, H, D, device="cuda"), torch.empty(333, H, D, device="cuda")
+    for _ in range(2):  # the first cache also loads the kernels
+        c = E.KvCache(1, KV, D, "f16", max_seq_len=ctx + 64, capacity=ctx + 64)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for S, at in ((100, 1000), (64, ctx), (333, 12001)):   # 8, 16 and 27.5 MiB of partials
+            E.attention(c, 0, q[:S], S, H, at, out=out[:S])
+        torch.cuda.synchronize()
+        used = free - torch.cuda.mem_get_info()[0]
+        c.close()
+    assert 33 << 20 <= used <= 35 << 20, used
