@@ -682,12 +682,19 @@ static int32_t ensure_workspace_floats(bg_kv_cache* c, size_t need, size_t count
   return BG_OK;
 }
 
+// Test hook: with BG_FAULT_PREFILL_ALLOC set the prefill's side buffers cannot be had.
+static hipError_t prefill_malloc(void** p, size_t bytes) {
+  if (!getenv("BG_FAULT_PREFILL_ALLOC")) return hipMalloc(p, bytes);
+  *p = nullptr;
+  return hipErrorOutOfMemory;
+}
+
 // Split-K prefill: the buffer of partials and their (m, l). False when it cannot be had (out of
 // memory, or the stream is being captured): the launch then scans whole key ranges, which needs none.
 static bool ensure_prefill_split(bg_kv_cache* c, hipStream_t st) {
   if (c->pf) return true;
   if (capturing(st)) return false;
-  if (hipMalloc((void**)&c->pf, bg::kPfSplitBytes + bg::kPfSplitMlBytes) != hipSuccess) {
+  if (prefill_malloc((void**)&c->pf, bg::kPfSplitBytes + bg::kPfSplitMlBytes) != hipSuccess) {
     (void)hipGetLastError();
     c->pf = nullptr;
   }
@@ -719,7 +726,7 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
   c->pf16 = nullptr;
   c->pf16_cap = 0;
   const size_t bytes = (size_t)(c->dtype == BG_KV_Q8 ? 2 : 1) * c->kv_heads * c->cap * c->D * sizeof(uint16_t);
-  hipError_t e = hipMalloc(&c->pf16, bytes);
+  hipError_t e = prefill_malloc(&c->pf16, bytes);
   if (e == hipSuccess) e = hipMemset(c->pf16, 0, bytes);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
@@ -734,14 +741,15 @@ static int32_t ensure_prefill_copy(bg_kv_cache* c) {
 int32_t bg_attention_reserve(bg_kv_cache* c, int32_t S, int32_t H) {
   if (!c || S < 1 || H < 1 || H % c->kv_heads) return fail(BG_E_INVALID, "bg_attention_reserve: bad arguments");
   if (c->dtype == BG_KV_F32 && !bg::f32_split_supported(view(c, 0), S, H)) {
-    if (c->D == 128 && !ensure_prefill_split(c, nullptr))
-      return fail(BG_E_OOM, "GPU out of memory during the split prefill workspace allocation");
+    // as for the launches: without the buffer they run in one part
+    if (c->D == 128) (void)ensure_prefill_split(c, nullptr);
     return BG_OK;
   }
   if (c->dtype != BG_KV_F32 && !bg::decode_preferred(view(c, 0), S, H)) {
     if (bg::prefill_wants_f16_copy(view(c, 0), S, H)) {
       int32_t rc = ensure_prefill_copy(c);
-      if (rc != BG_OK) return rc;
+      if (rc != BG_OK && !c->roll) return rc;  // sink mode: staged without it
+      if (rc != BG_OK) (void)hipGetLastError();
     }
     if (bg::prefill_can_split(view(c, 0), S, H, c->num_cus) &&
         !ensure_prefill_split(c, nullptr))

@@ -276,7 +276,9 @@ int32_t bg_attention_noalloc(bg_kv_cache* cache, int32_t layer, const float* q, 
  * attended slots, allocate that copy; for a prefill of S rows that can split along the key range, its partials
  * and (m, l) buffer. Call before capturing bg_attention into a HIP graph (a launch under capture
  * cannot allocate). A later call that needs a larger workspace allocates a new one and keeps the
- * old one until bg_kv_destroy, so launches captured before stay valid. */
+ * old one until bg_kv_destroy, so launches captured before stay valid. BG_E_OOM where a buffer
+ * cannot be had, except the partials of an f32 cache and the copy of a sink-mode one: launches run
+ * without these. */
 int32_t bg_attention_reserve(bg_kv_cache* cache, int32_t S, int32_t H);
 
 /* ---- sink-mode eviction (overflow 'sinks') ------------------------------------------------

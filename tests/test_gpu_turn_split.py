@@ -7,8 +7,10 @@ import pytest
 import torch
 
 from bitgpu_amd import engine as E
+from bitgpu_amd._lib import GpuOutOfMemoryError, check, lib
 from oracle import ref
 from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc, t
+from tests.test_gpu_sink_copy import _ring
 from tests.test_gpu_split_prefill import _case, _check
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +66,38 @@ def test_split_partials_stay_within_their_bound(dev):
         used = free - torch.cuda.mem_get_info()[0]
         c.close()
     assert 33 << 20 <= used <= 35 << 20, used
+
+
+def test_reserve_without_memory(dev, monkeypatch):
+    """Where an f32 or sink-mode launch can do without the partials and the copy, a reserve that
+    cannot have them is no error; f16 and q8 report it, and the plain q8 prefill, which needs its
+    copy, too."""
+    H, KV, D, ctx, S = 32, 8, 128, 2000, 150
+
+    def reserve(c, S):
+        check(lib().bg_attention_reserve(c.handle, S, H))
+    monkeypatch.setenv("BG_FAULT_PREFILL_ALLOC", "1")
+    c, _, q, _ = _case("f32", H, KV, D, ctx + S, S, seed=6, gate=False)
+    reserve(c, S)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    want = ref.attention(q, kk, vv, ctx)
+    assert np.abs(run_attention(c, 0, q, ctx) - want).max() <= 1e-4
+    c.close()
+    c, q, want = _ring("f16", H, KV, D, 1000, (300,), 700, 100, "slot")
+    # (the copy is let go; the partials of an f16 cache are reported as before)
+    with pytest.raises(GpuOutOfMemoryError, match="split prefill"):
+        reserve(c, 100)
+    _check(run_attention(c, 0, q, 700), want)
+    c.close()
+    c, _, q, _ = _case("q8", H, KV, D, 700, 60, seed=7, gate=False)
+    with pytest.raises(GpuOutOfMemoryError, match="split prefill"):
+        reserve(c, 60)
+    with pytest.raises(GpuOutOfMemoryError, match="f16 copy"):
+        reserve(c, 128)
+    kk, vv = cached_values(c, 0, 0, 700)
+    _check(run_attention(c, 0, q, 640), ref.attention(q, kk, vv, 640))
+    with pytest.raises(GpuOutOfMemoryError):
+        run_attention(c, 0, np.repeat(q, 3, 0), 500)
+    monkeypatch.delenv("BG_FAULT_PREFILL_ALLOC")
+    reserve(c, 128)
+    c.close()
