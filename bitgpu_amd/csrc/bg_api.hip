@@ -718,19 +718,17 @@ static int32_t ensure_workspace(bg_kv_cache* c, int S, int H) {
   return ensure_workspace_floats(c, need, counters);
 }
 
-// the f16 prefill copy holds one layer at the cache's physical capacity (zero-filled, so slots
-// past the dequantized range read as finite zeros)
+// the f16 prefill copy holds one layer at the cache's physical capacity. Not filled: a launch converts
+// every slot its steps read (whole 64-slot steps, up to the capacity), and a fill would have to wait
+// for the device, other streams' work included.
 static int32_t ensure_prefill_copy(bg_kv_cache* c) {
   if (c->pf16 && c->pf16_cap == c->cap) return BG_OK;
   if (c->pf16) (void)hipFree(c->pf16);
   c->pf16 = nullptr;
   c->pf16_cap = 0;
   const size_t bytes = (size_t)(c->dtype == BG_KV_Q8 ? 2 : 1) * c->kv_heads * c->cap * c->D * sizeof(uint16_t);
-  hipError_t e = prefill_malloc(&c->pf16, bytes);
-  if (e == hipSuccess) e = hipMemset(c->pf16, 0, bytes);
-  if (e == hipSuccess) e = hipDeviceSynchronize();
+  const hipError_t e = prefill_malloc(&c->pf16, bytes);
   if (e != hipSuccess) {
-    if (c->pf16) (void)hipFree(c->pf16);
     c->pf16 = nullptr;
     return hip_fail(e, "prefill f16 copy allocation");
   }

@@ -70,3 +70,37 @@ def test_sink_prefill_captured_without_reserve(dev):
         torch.cuda.synchronize()
         _check(out.cpu().numpy(), want)
     c.close()
+
+
+@pytest.mark.parametrize("dtype,kw", [("f16", dict(overflow="sinks", sink_tokens=4)), ("q8", {})])
+def test_first_copy_does_not_wait_for_other_streams(dev, dtype, kw):
+    """The first prefill of a cache allocates its copy and returns while another stream is busy
+    (with 40 products of 8192 x 8192 f32 matrices, a few hundred ms), and is right."""
+    H, KV, D, S = 32, 8, 128, 200
+    cos, sin, _, _ = rope_dev(1e6, D, 1024)
+    q = torch.randn(S, H, D, device="cuda")
+    k, v = (torch.randn(S, KV, D, device="cuda") for _ in range(2))
+    m = torch.randn(8192, 8192, device="cuda")
+    p = m @ m
+    outs = []
+    for busy in (False, True):  # the first round also loads the kernels
+        c = E.KvCache(1, KV, D, dtype, max_seq_len=1024, capacity=1024, **kw)
+        if kw:
+            c.set_rope(cos, sin)
+        c.append_kv(k, 0, 0, S * KV, 0)
+        c.append_kv(v, 1, 0, S * KV, 0)
+        out = torch.empty_like(q)
+        torch.cuda.synchronize()
+        other, done = torch.cuda.Stream(), torch.cuda.Event()
+        if busy:
+            with torch.cuda.stream(other):
+                for _ in range(40):
+                    torch.matmul(m, m, out=p)
+                done.record()
+        E.attention(c, 0, q, S, H, 0, out=out)
+        waited = done.query()
+        torch.cuda.synchronize()
+        assert not (busy and waited)
+        outs.append(out.clone())
+        c.close()
+    assert torch.equal(*outs)
