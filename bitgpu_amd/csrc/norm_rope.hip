@@ -124,7 +124,7 @@ struct RowLayout {
 // cos/sin row and holds it once (fewer registers: 8 waves a SIMD instead of 6)
 // NI row load instructions a wave. 4: workgroups of four waves, the items' kinds interleaved; 1 and 2:
 // a wave a workgroup, items in plain order (the interleaving costs five 64-bit divisions, longer
-// than a decode step's rows take to load). Which: prologue_ni.
+// than a decode step's rows take to load). Which: prologue_few.
 template <int D, int DT, bool SP, int NI>
 __global__ __launch_bounds__(NI == 4 ? 256 : 64) void qkv_prologue_kernel(LayerView L, PrologueArgs a, PrologueGrid gr) {
   using RL = RowLayout<D, NI>;
@@ -294,17 +294,14 @@ __global__ __launch_bounds__(NI == 4 ? 256 : 64) void qkv_prologue_kernel(LayerV
   }
 }
 
-// Load instructions of rows a wave. Few rows are bound by latency and spread over the most waves (a
-// decode step, 32 + 8 heads: 3.1 us, two 3.8, four 5.1; 64 positions 3.9, 4.5, 5.5). Many rows of
-// f16 or q8 keys are best two at a time in plain order (us for 2048 positions f16 / 4096 q8 / 8192
-// q8 at head_dim 256: 18.1 / 36.2 / 83.8, one 19.0 / 37.6 / 91, four interleaved 20.3 / 38.7 / 90);
-// f32 storage, whose V groups write twice the bytes, four interleaved (4096 positions 34.9, in
-// plain order 40; 1500 20.0 against 18.6 with one). The lines lie between the sizes measured: f16
-// and q8 2,560 rows (one) and 13,320 (8.0, two 7.3), f32 60,000 (one) and 98,000.
-static int prologue_ni(int dtype, long rows) {
-  if (rows <= (dtype == KV_F32 ? 65536 : 8192)) return 1;
-  return dtype == KV_F32 ? 4 : 2;
-}
+// Load instructions of rows a wave (NI). Few rows are bound by latency and spread over the most waves,
+// one load each (a decode step, 32 + 8 heads: 3.1 us, two 3.8, four 5.1; 64 positions 3.9, 4.5, 5.5).
+// Many rows of f16 or q8 keys are best two at a time in plain order (us for 2048 positions f16 / 4096
+// q8 / 8192 q8 at head_dim 256: 18.1 / 36.2 / 83.8, one 19.0 / 37.6 / 91, four interleaved 20.3 / 38.7
+// / 90); f32 storage, whose V groups write twice the bytes, four interleaved (4096 positions 34.9, in
+// plain order 40; 1500 20.0 against 18.6 with one). The lines between few and many lie between the
+// sizes measured: f16 and q8 2,560 rows (one) and 13,320 (8.0, two 7.3), f32 60,000 (one) and 98,000.
+static bool prologue_few(int dtype, long rows) { return rows <= (dtype == KV_F32 ? 65536 : 8192); }
 
 template <int D, int DT, int NI>
 static void launch_prologue(const LayerView& L, const PrologueArgs& a, const PrologueGrid& gr, hipStream_t st) {
@@ -340,7 +337,7 @@ static hipError_t prologue_d(const LayerView& L, const PrologueArgs& a, hipStrea
     }
     gr.nvs = a.S - 16 * gr.ng;
   }
-  const bool few = prologue_ni(L.dtype, (long)gr.nq + gr.nk) == 1;
+  const bool few = prologue_few(L.dtype, (long)gr.nq + gr.nk);
   switch (L.dtype) {
     case KV_F32:
       if (few) launch_prologue<D, KV_F32, 1>(L, a, gr, st);
