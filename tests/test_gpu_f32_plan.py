@@ -10,6 +10,7 @@ from oracle import ref
 from tests.gpu_helpers import cached_values, run_attention, run_attention_noalloc, t
 from tests.test_gpu_sink_copy import _ring
 from tests.test_gpu_split_prefill import _case
+from tests.test_host import f32_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +60,52 @@ def test_f32_sink_ring(dev, window, moves, fill, S, mode):
 def test_f32_sink_prompt_before_any_eviction(dev, H, KV, D, fill, S, mode):
     """The ring's origin has not moved: the causal bound, as for the plain cache."""
     c, q, want = _ring("f32", H, KV, D, 1000, (), fill, S, mode)
+    out = run_attention(c, 0, q, fill)
+    assert np.abs(out - want).max() <= 1e-4
+    assert np.array_equal(run_attention_noalloc(c, 0, q, fill), out)
+    c.close()
+
+
+def _plan(KV, S, H, pos_base, **ring):
+    """(waves sharing 32 rows, parts) and queries an item of the launch on this GPU."""
+    rc, (ks, QB, parts, _) = f32_plan(KV, S, H, pos_base, cus=torch.cuda.get_device_properties(0).multi_processor_count, **ring)
+    assert rc == 0
+    return (ks, parts), QB
+
+
+@pytest.mark.parametrize("H,KV,ctx,S,gate,ks,parts", [
+    (32, 8, 1000, 90, True, 1, 9),     # four row groups an item; the last item's groups end before its last part
+    (16, 4, 9000, 200, False, 1, 9),
+    (32, 8, 16000, 600, False, 1, 3),
+    (24, 8, 1500, 120, False, 1, 9),   # 3 heads a kv head: a query's rows in two groups
+    (24, 8, 800, 121, True, 2, 5),
+    (16, 2, 1000, 104, False, 2, 9),   # two row groups an item
+])
+def test_f32_row_groups_in_parts(dev, H, KV, ctx, S, gate, ks, parts):
+    """Waves of one or two row groups whose keys are split over workgroups, on a sample of the rows
+    (ends and row group borders among them)."""
+    plan, QB = _plan(KV, S, H, ctx)
+    assert plan == (ks, parts)
+    c, _, q, g = _case("f32", H, KV, 128, ctx + S, S, seed=ctx + S, gate=gate)
+    out = run_attention(c, 0, q, ctx, gate=g)
+    kk, vv = cached_values(c, 0, 0, ctx + S)
+    for r in sorted({0, 7, 8, 10, 11, QB - 1, QB, S // 2, S - 9, S - 2, S - 1}):
+        a = (q[r:r + 1], kk[:ctx + r + 1], vv[:ctx + r + 1])
+        want = ref.gated_attention(*a, g[r:r + 1], ctx + r) if gate else ref.attention(*a, ctx + r)
+        assert np.abs(out[r:r + 1] - want).max() <= 1e-4, r
+    assert np.isfinite(out).all() and np.array_equal(run_attention_noalloc(c, 0, q, ctx, gate=g), out)
+    c.close()
+
+
+@pytest.mark.parametrize("H,KV,window,moves,fill,S,mode,ks,parts", [
+    (32, 8, 1000, (300,), 225, 769, "slot", 1, 1),
+    (32, 8, 1000, (300,), 502, 321, "absolute", 2, 1),
+    (24, 4, 2000, (700,), 1911, 83, "slot", 1, 16),
+    (32, 8, 4096, (1500,), 4063, 27, "absolute", 2, 13),
+])
+def test_f32_ring_row_groups(dev, H, KV, window, moves, fill, S, mode, ks, parts):
+    c, q, want = _ring("f32", H, KV, 128, window, moves, fill, S, mode)
+    assert _plan(KV, S, H, fill, window=window + 4, sinks=4, head=c.ring_state()[0])[0] == (ks, parts)
     out = run_attention(c, 0, q, fill)
     assert np.abs(out - want).max() <= 1e-4
     assert np.array_equal(run_attention_noalloc(c, 0, q, fill), out)
