@@ -1,9 +1,9 @@
 """GPU: attention launches captured in a HIP graph and replayed.
 
-bg_attention_reserve sizes everything a shape needs (split-K workspace, the split prefill's (m, l)
-buffer, a q8 cache's f16 copy), so the launch can be captured; the captured kernels keep no state
-between launches except the workspace slots, which every launch leaves holding the empty marker
-(no memset is recorded: the kernels write the marker back themselves). Each graph is replayed
+bg_attention_reserve sizes everything a shape needs (the decode's split-K workspace, the split
+prefill's partials, a q8 cache's f16 copy), so the launch can be captured; the captured kernels keep
+no state between launches except the decode's workspace slots, which every launch leaves holding the
+empty marker (no memset is recorded: the kernels write the marker back themselves). Each graph is replayed
 several times with eager launches of other shapes on the same cache in between, and every replay
 must give the eager result bit for bit. The allocation-free entry point is captured the same way
 after its first (set-up) call ran eagerly."""
@@ -76,10 +76,13 @@ def test_graph_replay_matches_eager(dev, dtype, H, KV, D, L, S, gated):
     c.close()
 
 
-def test_graph_survives_workspace_growth(dev):
-    """A decode captured with only its own shape reserved; then an eager split-K prefill grows the
-    cache's workspace (a new, larger buffer): the captured decode keeps the buffer it was captured
-    with (the cache retires it instead of freeing it) and still replays to the eager result."""
+@pytest.mark.parametrize("rows", [2, 8])
+def test_graph_survives_workspace_growth(dev, rows):
+    """A decode captured with only its own shape reserved; then an eager launch that needs more: a
+    verify of 2 on the decode kernel, which grows the workspace (a new, larger buffer: the cache
+    retires the old one instead of freeing it), or of 8, a split-K prefill, which allocates its
+    partials. The captured decode keeps the buffer it was captured with and still replays to the
+    eager result."""
     H, KV, D, L = 24, 4, 256, 8200
     c, q, gate = _inputs("q8", H, KV, D, L, 1, True, seed=11)
     scale = 1.0 / 16
@@ -93,8 +96,8 @@ def test_graph_survives_workspace_growth(dev):
         with torch.cuda.graph(graph, stream=s):
             E.attention(c, 0, q, 1, H, L - 1, scale=scale, gate=gate, gate_stride=D, out=out)
     torch.cuda.synchronize()
-    q8 = t(np.random.default_rng(3).standard_normal((8, H, D)).astype(np.float32))
-    between = lambda: E.attention(c, 0, q8, 8, H, L - 8, scale=scale)   # split-K prefill: grows the workspace
+    qn = t(np.random.default_rng(3).standard_normal((rows, H, D)).astype(np.float32))
+    between = lambda: E.attention(c, 0, qn, rows, H, L - rows, scale=scale)
     _replay_and_check(graph, out, want, between)
     c.close()
 

@@ -36,9 +36,9 @@ def _check_gemv(got, x, sign, sc, resid=None):
 
 
 @pytest.mark.parametrize("K,N0,N1,N2", [(4096, 4096, 1024, 1024),    # Qwen3-8B qkv
-                                        (2560, 4096, 1024, 1024),    # Qwen3-4B qkv (K not a tile multiple)
+                                        (2560, 4096, 1024, 1024),    # Qwen3-4B qkv (five 512-weight steps)
                                         (4096, 12288, 12288, 0),     # gate | up
-                                        (5120, 1000, 0, 0)])         # partial tile, rows not a wave multiple
+                                        (5120, 1000, 0, 0)])         # ten steps, a partial 16-row tile
 def test_gemv_split_matches_oracle(dev, K, N0, N1, N2):
     rng = np.random.default_rng(K + N0)
     sign, sc = _weight(rng, N0 + N1 + N2, K)
@@ -53,9 +53,9 @@ def test_gemv_split_matches_oracle(dev, K, N0, N1, N2):
 
 @pytest.mark.parametrize("K,N", [(4096, 4096), (12288, 4096), (4096, 2560), (384, 77), (128, 64), (4224, 300), (12416, 200)])
 def test_gemv_resid_matches_oracle(dev, K, N):
-    """o_proj / down_proj with the residual (src/engine.ts:1547, matmul_resid_mr_sg.wgsl): rows
-    read through the nibble table (K <= 4096, down to a single scale block), through x staged in
-    LDS (4224 just past the table, 12288) and from memory (12416, past the staging)."""
+    """o_proj / down_proj with the residual (src/engine.ts:1547, matmul_resid_mr_sg.wgsl): one
+    512-weight step a wave on up to 8 waves (K <= 4096, down to a single scale block) and on up to 16
+    (4224, its last step one block), two steps a wave (12288; 12416, its last step one block)."""
     rng = np.random.default_rng(K * 3 + N)
     sign, sc = _weight(rng, N, K)
     x = rng.standard_normal(K).astype(np.float32)
@@ -79,19 +79,18 @@ def _qkv_case(dtype, H, KV, D, K, pos, seed, roll=False):
 @pytest.mark.parametrize("H,KV,D", [(32, 8, 128), (16, 8, 128), (8, 2, 256), (20, 2, 128), (24, 12, 128)])
 def test_qkv_proj_prologue_equals_unfused(dev, dtype, H, KV, D):
     """One launch (projection, Q norm+rope, K norm+rope into the cache, V append) equals the
-    projection followed by the prologue, bit for bit: q_out and every stored K / V byte.
-    (32, 8), (20, 2) and (24, 12) at D=128 run 24-row workgroups (heads across workgroup
-    boundaries; 256 / 128 / 256 workgroups, the Q/K/V boundaries at different places), the
-    others 32-row ones."""
+    projection followed by the prologue, bit for bit: q_out and every stored K / V byte. 32-row
+    workgroups, four a head at D=128 and eight at 256: 192, 128, 96, 96 and 192 of them, the Q/K/V
+    boundaries at different places. (8, 2) at D=256 does not fall into eight runs of whole heads,
+    so its raw rows are written through; the others' stay in an XCD's L2."""
     _fused_equals_unfused(dtype, H, KV, D, 4096)
 
 
 @pytest.mark.parametrize("K", [5120, 13312])
 @pytest.mark.parametrize("H,KV,D", [(32, 8, 128), (8, 2, 256)])
 def test_qkv_proj_prologue_equals_unfused_long_rows(dev, H, KV, D, K):
-    """The same beyond the nibble table's 4096-weight rows: x staged in LDS (K = 5120, three
-    2048-weight tiles, the last one partial) and x read from memory (K = 13312), on 24-row and
-    32-row workgroups."""
+    """The same past the 8 waves of a 4096-weight row: 10 waves of one 512-weight step (K = 5120)
+    and 13 of two (K = 13312, the loop of any number of steps), with both ways of the raw rows."""
     _fused_equals_unfused("q8", H, KV, D, K)
 
 
@@ -158,8 +157,8 @@ def test_qkv_proj_sink_mode_keys_unroped(dev):
 def test_decode_attention_block_steps(dev):
     """The fused decode attention block (src/engine.ts:1519-1547) over several consecutive tokens
     of a q8 cache in the Qwen3-4B shape (hidden 2560, 32 heads on 8 kv heads): qkv projection +
-    prologue, attention, o_proj + residual, against the oracle composite (the arrival counters
-    reset after every launch, so repeated launches stay correct)."""
+    prologue, attention, o_proj + residual, against the oracle composite (every launch leaves
+    the gather buffer holding the empty marker, so repeated launches stay correct)."""
     H, KV, D, HD, past, steps = 32, 8, 128, 2560, 300, 4
     rng = np.random.default_rng(9)
     sign, sc = _weight(rng, (H + 2 * KV) * D, HD)

@@ -4,9 +4,8 @@ many heads per kv head, a short prompt chunk after a long context) against the o
 Each (query block, kv head) item's key range is scanned in parts by separate workgroups, whose
 partials a second kernel merges by log-sum-exp (the gate applied after the merge). Tolerances as
 for every f16 / q8 attention: relative 2e-3 and cosine > 0.99999 against ``ref.attention`` /
-``ref.gated_attention`` over the stored values. The partials share the decode kernel's
-workspace, whose slots must hold the empty marker after every launch: a decode on the same
-cache right after a split prefill checks that."""
+``ref.gated_attention`` over the stored values. The partials lie in a buffer of their own: a decode
+on the same cache right after a split prefill checks that the decode's workspace is left alone."""
 import numpy as np
 import pytest
 
@@ -54,7 +53,7 @@ def test_hybrid_verify_split(dev, dtype, S):
 def test_chunk_after_long_context_split(dev, dtype):
     """A 64-row prompt chunk after 8000 cached positions (runPrefill segments,
     src/engine.ts:1705-1735) in the Qwen3-8B shape: 16 items split over many parts; then a decode
-    step on the same cache (the workspace must be back to empty slots)."""
+    step on the same cache (whose workspace must still hold empty slots)."""
     H, KV, D, P, S = 32, 8, 128, 8000, 64
     L = P + S + 1
     c, rng, q, _ = _case(dtype, H, KV, D, L, S, seed=77, gate=False)
@@ -76,8 +75,8 @@ def test_sink_segment_after_wrap_split(dev, dtype):
 
 
 def test_split_prefill_repeated_launches(dev):
-    """Consecutive split launches with different part counts on one cache reuse the workspace:
-    each launch's merge leaves every slot it read empty for the next."""
+    """Consecutive split launches with different part counts on one cache use one buffer: a launch
+    reads only the partials it wrote itself."""
     H, KV, D = 24, 4, 256
     L = 6000
     c, rng, _, _ = _case("q8", H, KV, D, L, 1, seed=5, gate=False)
