@@ -131,7 +131,7 @@ void free_layers(std::vector<void*>& k, std::vector<void*>& v, std::vector<float
   k.clear(); v.clear(); ks.clear(); vs.clear();
 }
 
-// heads (query + key + value) the fused decode projection's arrival counters cover
+// heads (query + key + value) the fused decode projection's gather buffer covers
 constexpr int kProjMaxHeads = 1024;
 
 // slots the caller may address: the window in sink mode, the grown capacity otherwise
@@ -646,8 +646,8 @@ int32_t bg_qkv_prologue(bg_kv_cache* c, int32_t layer, const float* q, int32_t q
 }
 
 // The attention workspace: decode or f32 split partials (each launch uses one kind; every slot
-// holds the empty marker between launches). Grows to at
-// least `need` floats and `counters` counters, keeping the larger of old and new.
+// holds the empty marker between launches). Grows to at least `need` floats and `counters`
+// counters, keeping the larger of old and new.
 static int32_t ensure_workspace_floats(bg_kv_cache* c, size_t need, size_t counters) {
   if (need < c->ws_floats) need = c->ws_floats;
   if (counters < c->ws_counters) counters = c->ws_counters;

@@ -84,9 +84,8 @@ struct QkvProjArgs {
 };
 // raw-row floats the fused projection's gather buffer holds (heads of every kind x head_dim)
 size_t qkv_proj_raw_floats(int heads, int D);
-// Arrival counters (the fused projection's per head, the f32 decode's per kv head) sit 256 bytes
-// apart: 384 workgroups' atomics on counters packed into two lines serialize (the 8B-shape qkv
-// projection took 8.6 us with them packed, 7.5 us apart).
+// Arrival counters (the f32 decode's, per kv head) sit 256 bytes apart: many workgroups' atomics on
+// counters packed into two lines serialize.
 constexpr int kCounterStride = 64;
 hipError_t launch_qkv_proj(const LayerView& L, const QkvProjArgs& a, hipStream_t st);
 
@@ -149,8 +148,8 @@ bool decode_plan(const LayerView& L, int S, int H, int pos_base, int num_cus, in
 hipError_t launch_stream_read(const void* buf, size_t bytes, int workgroups, bool nontemporal, unsigned* sink,
                               hipStream_t st);
 bool prefill_supported(const LayerView& L, int S, int H);
-// a q8 prefill of S rows that stages each K/V tile for enough query blocks to run faster on an
-// f16 copy of the attended slots
+// a q8 or sink-mode prefill of S rows that stages each K/V tile for enough query blocks to run faster
+// on an f16 copy of the attended slots
 bool prefill_wants_f16_copy(const LayerView& L, int S, int H);
 // "not written yet" marker of a split partial slot: a quiet NaN with a payload arithmetic on
 // finite inputs never produces. The decode kernel leaves every slot it uses holding it.

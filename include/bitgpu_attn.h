@@ -17,10 +17,12 @@
  *     one split workspace and one f16 prefill copy, so two bg_attention calls on different
  *     streams could overlap on the GPU and corrupt each other's partials.
  *   - Kernels never allocate. Host-side allocations happen only in bg_kv_create, bg_kv_grow,
- *     bg_attention_reserve, lazily on the first bg_attention that needs more workspace (split
- *     partials, at most 33 MiB of them for a split-K prefill, which runs unsplit where they cannot
- *     be had) or, for a q8 or sink-mode cache, the f16 copy a long prefill runs on, and in the snapshot
- *     transfers (a staging buffer kept by the cache, grown when a larger region is transferred).
+ *     bg_attention_reserve, lazily on the first bg_attention that needs more workspace (the
+ *     decode's split partials; 33 MiB for a split-K prefill's, which runs unsplit, in several times
+ *     the time, where it cannot have them, as in a capture that was not reserved for) or, for a q8 or
+ *     sink-mode cache, the f16 copy a long prefill runs on, and in the snapshot transfers (16 MiB of
+ *     pinned memory for the process; region by region a staging buffer kept by the cache, grown when
+ *     a larger region is transferred).
  *   - The decode kernel's split merge waits a bounded time for the partials of its own grid.
  *     If a wait gives up (the GPU shared with work that keeps the grid from running at once),
  *     that launch stores NaN and raises the cache's error word; the next bg_attention on the
@@ -273,8 +275,8 @@ int32_t bg_attention_noalloc(bg_kv_cache* cache, int32_t layer, const float* q, 
 
 /* Pre-size the split-K workspace for up to S query rows of H heads (otherwise sized on first
  * use), and for a q8 or sink-mode cache whose prefill of S rows runs on an f16 copy of the
- * attended slots, allocate that copy; for a prefill of S rows that can split along the key range, its partials
- * and (m, l) buffer. Call before capturing bg_attention into a HIP graph (a launch under capture
+ * attended slots, allocate that copy; for a prefill of S rows that can split along the key range
+ * (an f32 one at head_dim 128: any), the 33 MiB of its partials. Call before capturing bg_attention into a HIP graph (a launch under capture
  * cannot allocate). A later call that needs a larger workspace allocates a new one and keeps the
  * old one until bg_kv_destroy, so launches captured before stay valid. BG_E_OOM where a buffer
  * cannot be had, except the partials of an f32 cache and the copy of a sink-mode one: launches run
