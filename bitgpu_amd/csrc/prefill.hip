@@ -847,6 +847,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void prefill_kernel(PrefillP
   }
 }
 
+constexpr int kMergeLoaded = 32;  // parts whose columns prefill_merge_kernel loads all at once
+
 // Split-K merge: workgroup (item, wave, o slot) combines that slot of the wave's 32 rows over the
 // parts by log-sum-exp, applies the gate (gate_sigmoid.wgsl:13 form) and stores the output
 // float4s; the four 64-lane groups take every fourth part and meet through LDS. It only reads the
@@ -878,7 +880,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
   // up to 4 * PB parts: every part's (m, l) and partial column loaded before any is used (one
   // memory round trip instead of one per part and group; D=128 f16 verify S=5-12 12.6-13.9 ->
   // 11.6-13.0 us); same order and arithmetic as the loops past it
-  constexpr int PB = 8;
+  constexpr int PB = kMergeLoaded / 4;
   float mx = -INFINITY;
   float2 mlb[PB];
   float4 vb[PB];
@@ -1051,11 +1053,17 @@ static bool pf_mirror(const LayerView& L, int n_items, int num_cus) { return L.D
 // Split-K plan of a prefill launch. A grid of (query block, kv head) items that leaves CUs idle
 // (a user turn or verify after a long context) splits every item's key range into parts of at
 // least kPfMinPartSteps steps, at most one round of workgroups. The part count is the cheapest by
-// a cost model in microseconds, its constants measured: a step takes about 1 us of a CU, 2.1 us
-// where a D=128 CU runs two workgroups; a part's partial (32 KB a wave at D=256, 16 KB at D=128)
-// is written and read at about 4.5 TB/s, and the merge kernel adds about 5 us. So a short prompt stays whole
-// (S=500: 14.8 us, 31 split in two) and a turn of 333 tokens after 12,000 takes five parts (184 ->
-// 107 us; two 127, three 135), 300 after 3,000 at D=256 four (129 -> 68 us; two 86, eight 83).
+// a cost model in microseconds, its constants measured: a step takes about 1 us of a CU (1.12 where
+// it masks by a ring's logical slots, 3 where it rotates sink-mode keys: one query block, no copy;
+// such parts go down to 2 steps), 2.1 times that where a D=128 CU runs two workgroups; a part's partial (32 KB a wave at D=256, 16 KB at D=128) is
+// written and read at about 4.5 TB/s; the merge adds 2 us up to 8 parts, 3 past that (the kernel of
+// a workgroup a slot), and 2 + 0.1 a part past 32 (its parts no longer all loaded at once). So a
+// short prompt stays whole (S=500: 14.8 us, 31 split in two) and a turn of 333 tokens after 12,000
+// takes five parts (184 -> 107 us; two 127, three 135), 300 after 3,000 at D=256 four (129 -> 68 us;
+// two 86, eight 83). With a merge of 5 us whatever the parts (in 260 measured shapes 27 slower than
+// with the plan of at most 8 MiB of partials before it; now two, by 5 and 9 %), us: 60 tokens after
+// 3,000, 32 heads 20.7 -> 18.1, 17 after 12,000, 16 heads on 2 20.9 -> 17.9, 200 after 300, 8 heads on
+// 8 14.2 -> 12.5, 17 in a wrapped window of 700, 30 -> 18.6.
 // Both entry points use the same plan (the allocation-free one's scratch holds every plan's
 // partials), so their results are the same.
 constexpr int kPfMinPartSteps = 4;
@@ -1077,16 +1085,20 @@ static PfSplitPlan pf_split_plan(const LayerView& L, int S, int H, int pos_base,
   const int waves = std::min(4, (std::min(QB, S) * G + 31) / 32);
   const size_t part_bytes = (size_t)waves * 4 * (L.D / 32) * 64 * sizeof(float4);
   const size_t ml_bytes = (size_t)waves * 64 * sizeof(float2);
-  int P = std::min(std::min(per_cu * num_cus / n_items, steps_max / kPfMinPartSteps), kPfMaxParts);
+  const bool rotates = L.ring.roll && S <= QB;
+  const int least = rotates ? 2 : kPfMinPartSteps;
+  const float us_step = rotates ? 3.0f : L.ring.roll ? 1.12f : 1.0f;
+  int P = std::min(std::min(per_cu * num_cus / n_items, steps_max / least), kPfMaxParts);
   P = std::min(P, (int)(kPfSplitBytes / (part_bytes * n_items)));
   P = std::min(P, (int)(kPfSplitMlBytes / (ml_bytes * n_items)));
   const float us_part = 2.0f * part_bytes / 4.5e6f;
-  float best = steps_max * 1.0f;
+  float best = steps_max * us_step;
   if (n_items > num_cus) best *= 2.1f;
   for (int np = 2; np <= P; np++) {
     const int ps = (steps_max + np - 1) / np;
     if ((steps_max + ps - 1) / ps != np) continue;  // the same split as fewer parts
-    const float t = ps * (n_items * np > num_cus ? 2.1f : 1.0f) + n_items * np * us_part + 5.0f;
+    const float merge = (np <= kMergeParts ? 2.0f : 3.0f) + (np > kMergeLoaded ? 2.0f + 0.1f * np : 0.0f);
+    const float t = ps * us_step * (n_items * np > num_cus ? 2.1f : 1.0f) + n_items * np * us_part + merge;
     if (t < best) {
       best = t;
       r.n_parts = np;

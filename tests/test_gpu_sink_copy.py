@@ -55,6 +55,23 @@ def test_sink_prefill_copy_equals_staging(dev, dtype, D, window, moves, fill, S,
     c.close()
 
 
+@pytest.mark.parametrize("dtype,H,KV,D,window,moves,fill,S", [
+    ("f16", 32, 8, 128, 700, (200,), 350, 17),     # nine steps, room left out: three parts of three
+    ("q8", 32, 8, 128, 700, (), 660, 16),          # six parts of two steps, the last of one
+    ("f16", 16, 1, 128, 1500, (400,), 1400, 7),    # twelve parts: the merge of a workgroup a slot
+    ("q8", 24, 4, 256, 700, (600,), 350, 9),
+    ("f16", 64, 8, 128, 4096, (1500,), 4050, 16),  # 128 rows, parts of three
+])
+def test_one_block_in_parts_of_rotating_steps(dev, dtype, H, KV, D, window, moves, fill, S):
+    """One query block of more rows than the decode kernel takes: no copy, every step rotates its keys,
+    parts down to two steps."""
+    c, q, want = _ring(dtype, H, KV, D, window, moves, fill, S)
+    out = run_attention(c, 0, q, fill)
+    _check(out, want)
+    assert np.array_equal(run_attention_noalloc(c, 0, q, fill), out)
+    c.close()
+
+
 def test_sink_prefill_captured_without_reserve(dev):
     H, KV, D, fill, S = 32, 8, 128, 1500, 160
     c, q, want = _ring("f16", H, KV, D, 2000, (700,), fill, S)
