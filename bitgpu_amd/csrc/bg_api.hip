@@ -1076,9 +1076,9 @@ int32_t bg_f32_prefill_plan(int32_t kv_heads, int32_t S, int32_t H, int32_t pos_
   L.ring.W = L.max_seq - L.ring.sinks;
   L.ring.head = window ? head : 0;
   const bg::F32Plan p = bg::f32_plan(L, S, H, pos_base, num_cus, partials ? bg::kPfSplitBytes / sizeof(float) : 0);
-  if (!p.QB) return fail(BG_E_UNSUPPORTED, "bg_f32_prefill_plan: no plan for %d heads on %d", H, kv_heads);
+  if (H / kv_heads > 128) return fail(BG_E_UNSUPPORTED, "bg_f32_prefill_plan: %d heads on %d", H, kv_heads);
   out[0] = p.ks;
-  out[1] = p.QB;
+  out[1] = p.QB ? p.QB : 128 / (H / kv_heads);
   out[2] = p.n_parts;
   out[3] = p.part_steps;
   return BG_OK;

@@ -170,8 +170,9 @@ hipError_t launch_prefill_merge(const LayerView& L, const AttnArgs& a, int QB, i
 void prefill_skip(const LayerView& L, int S, int pos_base, int KT, int* t0, int* n);
 // The plan of an f32 prefill launch (host-only arithmetic): ks of a workgroup's four waves share 32
 // rows and take every ks-th 32-key step (4 / ks row groups an item), QB queries an item, n_parts
-// parts of part_steps 64-key steps, at most `floats` floats of partials. QB = 0: the kernel of 128-row
-// items staged through LDS (head_dim 256, whose K, V, Q and O a step would not fit a wave's registers).
+// parts of part_steps 64-key steps, at most `floats` floats of partials. ks = QB = 0: the kernel of
+// 128-row items staged through LDS (a single step of few rows; head_dim 256, whose K, V, Q and O a step
+// would not fit a wave's registers).
 struct F32Plan {
   int ks, QB, n_parts, part_steps;
 };

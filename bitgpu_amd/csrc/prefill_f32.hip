@@ -1,6 +1,6 @@
 // Causal GQA prefill over an f32 KV cache (kvCache 'f32', the reference default) on the f32
 // matrix cores of gfx950: prefill_f32_kernel at head_dim 256, prefill_f32_split_kernel (below) at
-// 128, the same arithmetic.
+// 128 past the shortest prompts, the same arithmetic.
 //
 // Replaces attention_sg.wgsl / attention_wg.wgsl (and their _roll and f32
 // attention_online_cache forms) for more than 16 rows per kv head: those run one subgroup per
@@ -569,6 +569,13 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_split_kernel(F32SplitParam
   if (sp.n_parts > 1 && ks == 0) sp.pml[pi * 64 + lane] = make_float2(M, lt);
 }
 
+// One 32-key step and at most 96 rows a kv head (a first prompt of a few words): the kernel above, whose
+// waves share the one step's K and V through LDS: 20 tokens, 16 heads on 8 9.2 us against 11.0, 32
+// on 8 10.0 / 10.9; 128 rows 11.0 / 11.0, 136 11.2 / 10.9; two steps 14.3 / 11.2.
+static bool f32_one_step(const LayerView& L, int S, int G, int pos_base) {
+  return !(L.ring.roll && L.ring.head != 0) && pos_base + S <= kF32KT && S * G <= 96;
+}
+
 // The cheapest by a cost model in us. A step takes 3.8 us of a wave (a CU runs one workgroup); an
 // item 2.5 to 4 before and after its steps. Where items are alike (a long context before the rows)
 // the grid runs in whole rounds of the CUs, else its longest item or its share of a CU counts,
@@ -578,9 +585,9 @@ __global__ __launch_bounds__(256, 1) void prefill_f32_split_kernel(F32SplitParam
 // what is cheapest in many parts is not (200 rows of 16 heads on 4 after 9,000 keys: nine parts of 128
 // rows, but in one part items of 32; captured without a buffer 1,155 -> 303 us).
 F32Plan f32_plan(const LayerView& L, int S, int H, int pos_base, int cus, size_t floats) {
-  F32Plan best{4, 0, 1, 0};
+  F32Plan best{0, 0, 1, 0};
   const int G = H / L.kv_heads;
-  if (L.D != 128 || G > 128) return best;
+  if (L.D != 128 || G > 128 || f32_one_step(L, S, G, pos_base)) return best;
   const bool fixed = L.ring.roll && L.ring.head != 0;
   int skip_t0, skip_n;
   prefill_skip(L, S, pos_base, 64, &skip_t0, &skip_n);
@@ -695,6 +702,7 @@ hipError_t launch_attention_f32(const LayerView& L, const AttnArgs& a, hipStream
   const int cus = a.num_cus > 0 ? a.num_cus : 256;
   p.mirror = 0;
   const bool roll = L.ring.roll != 0;
+  if (L.D == 128 && f.ks == 0) return roll ? launch_pf32<128, true>(p, grid, cus, st) : launch_pf32<128, false>(p, grid, cus, st);
   if (L.D == 256) return roll ? launch_pf32<256, true>(p, grid, cus, st) : launch_pf32<256, false>(p, grid, cus, st);
   return hipErrorInvalidValue;
 }

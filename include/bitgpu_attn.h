@@ -107,7 +107,8 @@ int32_t bg_decode_plan(int32_t kv_heads, int32_t head_dim, int32_t dtype, int32_
                        int32_t pos_base, int32_t num_cus, int32_t resident_per_cu, int32_t* out);
 
 /* The same for the f32 prefill at head_dim 128: out[0..3] = waves of a workgroup (of four) that
- * share 32 rows, queries per workgroup, parts the key range is split into, 64-key steps per part.
+ * share 32 rows (0: each its own rows, the keys shared through LDS, one part), queries per workgroup,
+ * parts the key range is split into, 64-key steps per part.
  * window > 0: a sink-mode ring of that many slots with `sinks` sinks and origin `head`; partials 0:
  * a launch that has no buffer for split partials. */
 int32_t bg_f32_prefill_plan(int32_t kv_heads, int32_t S, int32_t H, int32_t pos_base, int32_t window,

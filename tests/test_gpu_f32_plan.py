@@ -16,7 +16,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,KV,ctx,S,gate", [
-    (16, 8, 0, 9, False),       # 18 rows a kv head: one partial 32-row item
+    (16, 8, 0, 9, False),       # 18 rows a kv head over one step: 128-row items, keys through LDS
+    (16, 8, 24, 9, True),       # one more key than a step: a partial 32-row item
+    (12, 4, 0, 32, True),       # 96 rows over one step: the most that kernel takes
+    (16, 4, 7, 25, False),      # 100 rows over one step: 32-row items
     (16, 8, 0, 333, True),      # 32-row items, a ragged end
     (24, 8, 0, 129, False),     # 3 heads a kv head: queries across row groups
     (12, 1, 700, 40, False),    # 12 heads a kv head

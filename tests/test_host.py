@@ -267,6 +267,10 @@ def test_f32_plan_without_partials():
     assert f32_plan(4, 200, 16, 9000)[1][:3] == [1, 32, 9]
     assert f32_plan(4, 200, 16, 9000, partials=0)[1][:3] == [4, 8, 1]
     assert f32_plan(8, 600, 32, 16000)[1][:3] == [1, 32, 3]
+    # one 32-key step of few rows: 128-row items, keys shared through LDS
+    assert f32_plan(8, 20, 16, 0)[1][:3] == [0, 64, 1] and f32_plan(4, 32, 12, 0)[1][:3] == [0, 42, 1]
+    assert f32_plan(8, 20, 16, 13)[1][0] == 4 and f32_plan(4, 25, 16, 7)[1][0] == 4
+    assert f32_plan(8, 20, 16, 0, window=1004, sinks=4, head=300)[1][0] == 4  # a moved origin: the whole ring
     assert f32_plan(1, 3, 200, 0)[0] == _lib.BG_E_UNSUPPORTED  # more than 128 heads a kv head
     assert f32_plan(8, 3, 32, 1000, window=1000, sinks=4)[0] == _lib.BG_E_INVALID
 
