@@ -298,10 +298,17 @@ __global__ __launch_bounds__(NI == 4 ? 256 : 64) void qkv_prologue_kernel(LayerV
 // one load each (a decode step, 32 + 8 heads: 3.1 us, two 3.8, four 5.1; 64 positions 3.9, 4.5, 5.5).
 // Many rows of f16 or q8 keys are best two at a time in plain order (us for 2048 positions f16 / 4096
 // q8 / 8192 q8 at head_dim 256: 18.1 / 36.2 / 83.8, one 19.0 / 37.6 / 91, four interleaved 20.3 / 38.7
-// / 90); f32 storage, whose V groups write twice the bytes, four interleaved (4096 positions 34.9, in
-// plain order 40; 1500 20.0 against 18.6 with one). The lines between few and many lie between the
-// sizes measured: f16 and q8 2,560 rows (one) and 13,320 (8.0, two 7.3), f32 60,000 (one) and 98,000.
-static bool prologue_few(int dtype, long rows) { return rows <= (dtype == KV_F32 ? 65536 : 8192); }
+// / 90). f32 storage, whose V groups write twice the bytes, runs few rows until those bound it, then
+// four interleaved, the V writes spread under the rows: V of 12,000 rows of 128 floats (1500 positions of
+// 8 heads, 16 / 24 / 32 query heads 14.3 / 16.4 / 18.5 us, four 15.2 / 16.8 / 19.1), 16,384 (2048: 18.9 /
+// 21.3 / 24.0, four 18.4 / 21.1 / 24.1; at head_dim 256 37.3 / 36.3); K and V alone, 2400 positions 14.9 /
+// 13.9, at head_dim 256 24.3 / 20.0. Q alone is the same work for every storage type and runs as f32's
+// (8192 positions of 32 heads 45, two at a time 48.5). The lines lie between the sizes measured: f16
+// and q8 2,560 Q and K rows (one) and 13,320 (8.0, two 7.3), f32 without V 60,000 (one) and 98,000.
+static bool prologue_few(int dtype, const LayerView& L, const PrologueArgs& a, long rows) {
+  if (dtype == KV_F32 && a.v) return (long)a.S * L.kv_heads * L.D <= 14000L * 128;
+  return rows <= (dtype == KV_F32 ? 65536 : 8192);
+}
 
 template <int D, int DT, int NI>
 static void launch_prologue(const LayerView& L, const PrologueArgs& a, const PrologueGrid& gr, hipStream_t st) {
@@ -337,8 +344,9 @@ static hipError_t prologue_d(const LayerView& L, const PrologueArgs& a, hipStrea
     }
     gr.nvs = a.S - 16 * gr.ng;
   }
-  const bool few = prologue_few(L.dtype, (long)gr.nq + gr.nk);
-  switch (L.dtype) {
+  const int dtype = a.k || a.v ? L.dtype : (int)KV_F32;
+  const bool few = prologue_few(dtype, L, a, (long)gr.nq + gr.nk);
+  switch (dtype) {
     case KV_F32:
       if (few) launch_prologue<D, KV_F32, 1>(L, a, gr, st);
       else launch_prologue<D, KV_F32, 4>(L, a, gr, st);

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
     ("q8", 12, 3, 128, 96, 549, False),     # rows that share no position a wave; a width through LDS
     ("q8", 24, 4, 256, 64, 293, False),
     ("f16", 32, 8, 128, 128, 211, True),
-    ("f32", 24, 8, 128, 128, 2049, False),  # past f32's line (65,536 rows)
+    ("f32", 24, 8, 128, 128, 2049, False),  # past f32's line (1.8 M values of V)
+    ("f32", 12, 3, 256, 64, 2341, False),
 ])
 def test_layouts_give_the_same_bits(dev, dtype, H, KV, D, rot, S, roll):
     rng = np.random.default_rng(S)
@@ -35,3 +36,20 @@ def test_layouts_give_the_same_bits(dev, dtype, H, KV, D, rot, S, roll):
     assert torch.equal(whole.view(torch.int32), torch.cat(parts).view(torch.int32))
     assert caches[0].save_snapshot(S + p) == caches[1].save_snapshot(S + p)
     [c.close() for c in caches]
+
+
+@pytest.mark.parametrize("dtype,H,D,S", [("f16", 32, 128, 300), ("q8", 24, 256, 2800), ("f32", 32, 128, 2100)])
+def test_queries_alone(dev, dtype, H, D, S):
+    """Q without K and V, on few and many rows of every storage type: the bits of the whole call, and
+    nothing written to the cache."""
+    c = E.KvCache(1, 4, D, dtype, max_seq_len=S, capacity=S)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(S, h, D, generator=g, device="cuda") for h in (H, 4, 4))
+    gamma = torch.rand(D, generator=g, device="cuda") + 0.5
+    cos, sin, _, _ = rope_dev(1e6, D, S)
+    before = c.save_snapshot(S)
+    alone = E.qkv_prologue(c, 0, q, None, None, S, H, gamma, None, 1e-6, cos, sin, D, 0, 0)
+    assert c.save_snapshot(S) == before
+    whole = E.qkv_prologue(c, 0, q, k, v, S, H, gamma, gamma, 1e-6, cos, sin, D, 0, 0)
+    assert torch.equal(alone.view(torch.int32), whole.view(torch.int32))
+    c.close()
