@@ -100,7 +100,7 @@ def test_first_copy_does_not_wait_for_other_streams(dev, dtype, kw):
     m = torch.randn(8192, 8192, device="cuda")
     p = m @ m
     outs = []
-    for busy in (False, True):  # the first round also loads the kernels
+    for busy in (False, True):  # the first pass also loads the kernels
         c = E.KvCache(1, KV, D, dtype, max_seq_len=1024, capacity=1024, **kw)
         if kw:
             c.set_rope(cos, sin)
